@@ -8,6 +8,15 @@ namespace k3kda {
 
 // y[T][out] = W[out][in] . x[T][in] with double accumulation; wdt = K3_WF32 | K3_WBF16.
 int proj(int T, int in, int out, const float *x, const void *W, int wdt, float *y, hipStream_t st);
+// The same for up to PROJ_SEGS matrices W [rows][in] over one x in one launch, each into its
+// own y [T][rows].
+constexpr int PROJ_SEGS = 6;
+struct ProjSeg {
+    const void *W;
+    float *y;
+    int rows;
+};
+int proj_multi(int T, int in, const ProjSeg *segs, int n, const float *x, int wdt, hipStream_t st);
 
 // Row-major C[M][N] = A[M][K] . op(B) with fp32 accumulation (hipBLASLt): op(B) = B^T for
 // B [N][K] (b_trans) or B for B [K][N]; A and B both bf16 or both fp32; C bf16 or fp32;
@@ -156,6 +165,14 @@ int layer_step(int B, int H, int D, int K, float lb, float eps, float q_scale, c
                const float *q_conv, const float *k_conv, const float *v_conv, const float *A_log,
                const float *dt_bias, const float *o_norm, float *states, long stride, float *y,
                float *zout, long zn, hipStream_t st);
+
+// The core form (k3hip_kda_decode_step) for one sequence on fp32 inputs, with K4's mean of
+// squares summed across lanes in double and its root and division exact, as
+// k3hip_kda_epilogue computes them (the decode step itself adds the lanes in fp32).
+int step_exact(int H, int D, int K, float lb, float eps, float q_scale, const float *qi, const float *ki,
+               const float *vi, const float *z, const float *bl, const float *gate, const float *q_conv,
+               const float *k_conv, const float *v_conv, const float *A_log, const float *dt_bias,
+               const float *o_norm, float *hist, float *S, float *y, hipStream_t st);
 
 // p[0..n) = 0 on `st` with a kernel (never a memset node).
 int zero_fill(float *p, size_t n, hipStream_t st);

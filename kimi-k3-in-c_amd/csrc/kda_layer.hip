@@ -330,21 +330,37 @@ extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out
     const int E = w->hidden, H = w->H, D = w->D, K = w->K;
     const size_t P = (size_t)H * D, TP = (size_t)T * P;
 
-    // device intermediates, stream-ordered: qp kp vp z gl | q k v g alpha o y | bl beta | fa
-    const size_t nf = 12 * TP + 2 * (size_t)T * H + (size_t)T * D + (state ? 0 : (size_t)H * D * D);
+    // What runs between the projections and o_proj: for D = 64 / 128, one token as one launch
+    // (kda_step.hip) and a gate the chunked form takes as K1 fused into K2 and K4; otherwise K1,
+    // the recurrence and K4 one after another
+    // (calls beyond K1's limits go to it, to be refused there).
+    const bool wide = (D == 64 || D == 128) && H <= 65535 && T <= 65535L * 64;
+    const bool step = T == 1 && wide && K >= 1 && K <= 4;
+    const bool fused = T > 1 && wide && chunk_ready() && chunk_gate_ok(w->gate_lb);
+
+    // device intermediates, stream-ordered: qp kp vp z gl o y | q k v g alpha (unfused) | bl beta | fa |
+    // S and the conv history of a call without a state
+    const size_t TH = ((size_t)T * H + 3) & ~(size_t)3;   // fa starts 16-byte aligned
+    const size_t nS = state ? 0 : (size_t)H * D * D, nh = step && !state ? 3 * P * (size_t)(K - 1) : 0;
+    const size_t nf = (step || fused ? 7 : 12) * TP + nS + nh + 2 * TH + (size_t)T * D;
     StreamBuf ws;
     int rc = stream_alloc(ws, nf * sizeof(float), st);
     if (rc) return rc;
     float *f = (float *)ws.p;
-    float *qp = f, *kp = qp + TP, *vp = kp + TP, *z = vp + TP, *gl = z + TP;
-    float *q = gl + TP, *k = q + TP, *v = k + TP, *g = v + TP, *al = g + TP, *o = al + TP;
-    float *y = o + TP, *bl = y + TP, *bt = bl + (size_t)T * H, *fa = bt + (size_t)T * H;
-    float *S = state;
-    if (!S) {
-        S = fa + (size_t)T * D;
-        if ((rc = zero_fill(S, (size_t)H * D * D, st))) return rc;
+    float *qp = f, *kp = qp + TP, *vp = kp + TP, *z = vp + TP, *gl = z + TP, *o = gl + TP, *y = o + TP;
+    float *q = y + TP, *k = q, *v = q, *g = q, *al = q, *S = q;   // q .. alpha only where K1 runs on its own
+    if (!step && !fused) {
+        k = q + TP; v = k + TP; g = v + TP; al = g + TP;
+        S = al + TP;
     }
-    float *cs = state ? state + (size_t)H * D * D : nullptr;
+    float *cs = S + nS, *bl = cs + nh, *bt = bl + TH, *fa = bt + TH;
+    if (state) {
+        S = state;
+        cs = state + (size_t)H * D * D;
+    } else {
+        if ((rc = zero_fill(S, nS + nh, st))) return rc;
+        if (!step) cs = nullptr;
+    }
 
     // Projections. bf16 weights on a T >= 16 prefill: MFMA GEMMs (kda_mm.hip) of the input
     // split into bf16 hi + lo rows, the two halves' fp32 products added, so the products keep
@@ -369,30 +385,41 @@ extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out
         int r = mm(2 * T, nout, nin, K3HIP_BF16, xs, nin, W, nin, C2, K3HIP_F32, nout, st);
         return r ? r : pair_add(C2, y, T, nout, st);
     };
-    if (mfma && (rc = split_rows2(x, xs, T, E, st))) return rc;
-    if ((rc = project(E, (int)P, x, w->q, qp))) return rc;
-    if ((rc = project(E, (int)P, x, w->k, kp))) return rc;
-    if ((rc = project(E, (int)P, x, w->v, vp))) return rc;
-    if ((rc = project(E, H, x, w->b, bl))) return rc;
-    if ((rc = project(E, D, x, w->f_a, fa))) return rc;
-    if ((rc = project(E, (int)P, x, w->g, gl))) return rc;
-    if (mfma && (rc = split_rows2(fa, xs, T, D, st))) return rc;
+    if (mfma) {
+        if ((rc = split_rows2(x, xs, T, E, st))) return rc;
+        if ((rc = project(E, (int)P, x, w->q, qp))) return rc;
+        if ((rc = project(E, (int)P, x, w->k, kp))) return rc;
+        if ((rc = project(E, (int)P, x, w->v, vp))) return rc;
+        if ((rc = project(E, H, x, w->b, bl))) return rc;
+        if ((rc = project(E, D, x, w->f_a, fa))) return rc;
+        if ((rc = project(E, (int)P, x, w->g, gl))) return rc;
+        if ((rc = split_rows2(fa, xs, T, D, st))) return rc;
+    } else {
+        const ProjSeg in[6] = {{w->q, qp, (int)P}, {w->k, kp, (int)P}, {w->v, vp, (int)P},
+                               {w->g, gl, (int)P}, {w->f_a, fa, D},    {w->b, bl, H}};
+        if ((rc = proj_multi(T, E, in, 6, x, w->wdt, st))) return rc;
+    }
     if ((rc = project(D, (int)P, fa, w->f_b, z))) return rc;
 
-    if ((rc = k3hip_kda_prep(T, H, D, K, w->gate_lb, K3HIP_F32, qp, kp, vp, z, bl, w->q_conv,
-                             w->k_conv, w->v_conv, w->A_log, w->dt_bias, cs, q, k, v, g, al, bt,
-                             stream)))
-        return rc;
     const float qscale = 1.0f / sqrtf((float)D);
-    if (T == 1)
-        rc = k3hip_kda_decode(1, H, D, S, o, q, k, v, al, bt, qscale, stream);
-    else if (chunk_ready() && chunk_gate_ok(w->gate_lb) && (D == 64 || D == 128))
-        rc = k3hip_kda_chunk(T, H, D, 64, q, k, v, g, bt, qscale, S, o, nullptr, 0, stream);
-    else
-        rc = k3hip_kda_recurrent(T, H, D, q, k, v, al, bt, qscale, S, o, stream);
-    if (rc) return rc;
-    if ((rc = k3hip_kda_epilogue(T, H, D, w->rms_eps, o, gl, K3HIP_F32, w->o_norm, y, K3HIP_F32,
+    if (step) {
+        rc = step_exact(H, D, K, w->gate_lb, w->rms_eps, qscale, qp, kp, vp, z, bl, gl, w->q_conv, w->k_conv,
+                        w->v_conv, w->A_log, w->dt_bias, w->o_norm, cs, S, y, st);
+    } else if (fused) {
+        rc = k3hip_kda_prefill(T, H, D, K, w->gate_lb, K3HIP_F32, qp, kp, vp, z, bl, w->q_conv, w->k_conv,
+                               w->v_conv, w->A_log, w->dt_bias, cs, qscale, S, o, nullptr, 0, stream);
+    } else {
+        if ((rc = k3hip_kda_prep(T, H, D, K, w->gate_lb, K3HIP_F32, qp, kp, vp, z, bl, w->q_conv,
+                                 w->k_conv, w->v_conv, w->A_log, w->dt_bias, cs, q, k, v, g, al, bt,
                                  stream)))
+            return rc;
+        if (T == 1)
+            rc = k3hip_kda_decode(1, H, D, S, o, q, k, v, al, bt, qscale, stream);
+        else
+            rc = k3hip_kda_recurrent(T, H, D, q, k, v, al, bt, qscale, S, o, stream);
+    }
+    if (rc) return rc;
+    if (!step && (rc = k3hip_kda_epilogue(T, H, D, w->rms_eps, o, gl, K3HIP_F32, w->o_norm, y, K3HIP_F32, stream)))
         return rc;
     if (mfma && (rc = split_rows2(y, xs, T, (int)P, st))) return rc;
     return project((int)P, E, y, w->o, out);

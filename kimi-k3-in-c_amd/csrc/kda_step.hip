@@ -75,6 +75,7 @@ struct StepArgs {
     float *zout;                // zn floats zeroed on the way (may be nullptr)
     long zn;
     int stream_state;           // 1: nontemporal state loads and stores
+    int exact_norm;             // 1: K4's mean of squares in double across lanes (layer_dev)
 };
 
 template <int D, int K, bool ZIN>
@@ -294,7 +295,15 @@ __global__ __launch_bounds__(4 * D) void kda_layer_step_kernel(const StepArgs a)
 #pragma unroll
         for (int r = 1; r < RPP; r++) x = x + s_opart[r][tid < CPR ? tid : 0];
         const float part = tid < CPR ? ((x.x * x.x) + (x.y * x.y)) + ((x.z * x.z) + (x.w * x.w)) : 0.0f;
-        const float inv = __builtin_amdgcn_rsqf(half_wave_sum(part) / (float)D + a.eps);
+        float inv;
+        if (ZIN && a.exact_norm) {   // kda_epilogue2_kernel's arithmetic
+            double ss = (double)part;
+#pragma unroll
+            for (int m = 16; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+            inv = (float)(1.0 / sqrt(ss / (double)D + (double)a.eps));
+        } else {
+            inv = __builtin_amdgcn_rsqf(half_wave_sum(part) / (float)D + a.eps);
+        }
         if (tid < CPR) {
             f4 out;
 #pragma unroll
@@ -369,6 +378,29 @@ int layer_step(int B, int H, int D, int K, float lb, float eps, float q_scale, c
     a.zout = zout; a.zn = zn;
     a.stream_state = (size_t)B * P * D * 4 > STATE_CACHED_BYTES;
     return launch_step_d<false>(D, K, B, a, st);
+}
+
+int step_exact(int H, int D, int K, float lb, float eps, float q_scale, const float *qi, const float *ki,
+               const float *vi, const float *z, const float *bl, const float *gate, const float *q_conv,
+               const float *k_conv, const float *v_conv, const float *A_log, const float *dt_bias,
+               const float *o_norm, float *hist, float *S, float *y, hipStream_t st)
+{
+    if (((uintptr_t)S | (uintptr_t)gate | (uintptr_t)y | (uintptr_t)o_norm) & 15)
+        K3_FAIL(K3HIP_EINVAL, "decode step: S, gate, y and o_norm must be 16-byte aligned");
+    const size_t P = (size_t)H * D;
+    StepArgs a{};
+    a.H = H; a.lb = lb; a.eps = eps; a.q_scale = q_scale;
+    a.qi = qi; a.ki = ki; a.vi = vi; a.ldi = (long)P; a.in_dt = K3HIP_F32;
+    a.bl = bl; a.ldb = H;
+    a.z = z; a.ldz = (long)P;
+    a.gl = gate; a.g_dt = K3HIP_F32; a.gsplit = 1;
+    a.q_conv = q_conv; a.k_conv = k_conv; a.v_conv = v_conv; a.A_log = A_log; a.dt_bias = dt_bias; a.o_norm = o_norm;
+    a.S = S; a.s_stride = (long)(P * D);
+    a.hist = hist; a.h_stride = (long)(3 * P * (size_t)(K - 1));
+    a.y = y; a.y_dt = K3HIP_F32;
+    a.stream_state = P * D * 4 > STATE_CACHED_BYTES;
+    a.exact_norm = 1;
+    return launch_step_d<true>(D, K, 1, a, st);
 }
 
 }  // namespace k3kda
