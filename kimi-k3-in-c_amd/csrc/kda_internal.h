@@ -73,13 +73,27 @@ int decode_strided(int B, int H, int D, float *S, long s_stride, float *o, const
                    const float *k, const float *v, const float *alpha, const float *beta,
                    float qs, hipStream_t st);
 
-// Stream-ordered scratch: hipMallocAsync on `st`, freed with hipFreeAsync on the same stream.
+// Stream-ordered scratch of one call: a block kept between calls (kda_layer.hip) or
+// hipMallocAsync on `st`, given back in stream order when the StreamBuf goes.
+struct WsBlock {
+    void *p;
+    size_t size;
+    int dev;
+    hipStream_t last;   // stream of its last call
+    hipEvent_t ev;      // after that call; none for the null stream
+    bool busy;
+};
+void ws_return(WsBlock *k, hipStream_t st);
+// A weight set was uploaded (+1) or released (-1); blocks are kept only while any is there.
+void ws_handles(int d);
 struct StreamBuf {
     void *p = nullptr;
     hipStream_t st = nullptr;
+    WsBlock *kept = nullptr;
     ~StreamBuf()
     {
-        if (p) (void)hipFreeAsync(p, st);
+        if (kept) ws_return(kept, st);
+        else if (p) (void)hipFreeAsync(p, st);
     }
 };
 int stream_alloc(StreamBuf &b, size_t bytes, hipStream_t st);

@@ -313,6 +313,7 @@ extern "C" int k3hip_mla_release(k3hip_mla_weights *w)
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     free(w);
+    ws_handles(-1);
     return K3HIP_OK;
 }
 
@@ -333,6 +334,7 @@ extern "C" int k3hip_mla_upload(const K3MlaW *w, const K3Cfg *c, k3hip_mla_weigh
                 c->hidden, c->q_lora, c->n_heads * c->v_head);
     k3hip_mla_weights *d = (k3hip_mla_weights *)calloc(1, sizeof *d);
     if (!d) K3_FAIL(K3HIP_ENOMEM, "k3hip_mla_upload: host allocation");
+    ws_handles(1);
     d->E = c->hidden; d->H = c->n_heads; d->QL = c->q_lora; d->KL = c->kv_lora;
     d->QN = c->qk_nope; d->QR = c->qk_rope; d->VH = c->v_head; d->gate = c->mla_out_gate && w->g;
     d->eps = c->rms_eps;

@@ -157,35 +157,52 @@ def _check(rc: int) -> None:
 
 
 # ------------------------------------------------------------- torch plumbing ----
+# A call's host time is most of a one-launch decode step (11 us of arguments and stream lookup
+# against 6 us of kernel), so these stay short: addresses as plain integers, the raw handle of
+# the current stream (the Stream object costs 3 us to build).
 def _ptr(t):
     """Device pointer of a torch tensor (None -> NULL). Refuses host tensors and
     non-contiguous views: the kernels index dense row-major memory."""
     if t is None:
         return None
     if isinstance(t, _DevPtr):
-        return C.c_void_p(t.addr)
+        return t.addr
     if not t.is_cuda:
         raise ValueError("k3kda: device tensor required")
     if not t.is_contiguous():
         raise ValueError("k3kda: contiguous tensor required")
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+_raw_stream = None
 
 
 def _stream(stream):
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    global _raw_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None:
+        import torch
+        torch.cuda.current_stream()   # initialises the device
+        get, dev = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+        if get and dev:
+            _raw_stream = lambda: get(dev())
+        else:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream
+    return _raw_stream()
+
+
+_DT = {}
 
 
 def _dt(t) -> int:
-    import torch
-    if t.dtype == torch.float32:
-        return F32
-    if t.dtype == torch.bfloat16:
-        return BF16
-    if t.dtype == torch.float16:
-        return F16
-    raise ValueError(f"k3kda: dtype {t.dtype} not supported (float32, bfloat16 or float16)")
+    if not _DT:
+        import torch
+        _DT.update({torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16})
+    try:
+        return _DT[t.dtype]
+    except KeyError:
+        raise ValueError(f"k3kda: dtype {t.dtype} not supported (float32, bfloat16 or float16)") from None
 
 
 def proj_gemm(a, b, c, stream=None) -> None:
