@@ -50,6 +50,15 @@ __device__ __forceinline__ uint16_t f2bf(float f)
     return (uint16_t)(u >> 16);
 }
 
+// x = p[0] + p[1] + p[2], bf16 bits, each the rounding error of the ones before it.
+__device__ __forceinline__ void split3(float x, uint16_t (&p)[3])
+{
+    p[0] = f2bf(x);
+    const float r = x - bf2f(p[0]);
+    p[1] = f2bf(r);
+    p[2] = f2bf(r - bf2f(p[1]));
+}
+
 // Load element i of an activation that is fp32 (dtype 0) or bf16 (dtype 1).
 template <int DT>
 __device__ __forceinline__ float load_act(const void *p, size_t i)

@@ -65,6 +65,8 @@ int epilogue_split(int T, int H, int D, float eps, const float *o, const void *g
 // x [B][N] fp32 -> y [2B][N] bf16: rows 0..B-1 = hi, rows B..2B-1 = lo = bf16(x - hi), the
 // input of a GEMM that reads each weight once for both halves.
 int split_rows2(const float *x, uint16_t *y, int B, int N, hipStream_t st);
+// The same into three planes y [3B][N], x = hi + mid + lo with all its 24 bits.
+int split_rows3(const float *x, uint16_t *y, int B, int N, hipStream_t st);
 // y[b][n] = C2[b][n] + C2[B+b][n] (the two halves of such a GEMM).
 int pair_add(const float *C2, float *y, int B, int N, hipStream_t st);
 
@@ -105,7 +107,7 @@ size_t rows_frag_elems(int N, int K);
 int rows_frag_pack(const uint16_t *W, int N, int K, uint16_t *Wf, hipStream_t st);
 
 // C[B][N] (row stride ldc) = x[B][K] (fp32, row stride ldx) . W[N][K]^T (bf16, given as its
-// fragment-ordered copy Wf from rows_frag_pack), each x element split into bf16 hi + lo in
+// fragment-ordered copy Wf from rows_frag_pack), each x element split into bf16 hi + mid + lo in
 // registers so products keep fp32 accuracy; built for few rows (decode batches), bound by
 // reading W once. K % 8 == 0, ldx % 4 == 0, x and Wf 16-byte aligned. Stream-ordered.
 // Split-K partials go to ws (16-byte aligned, at least gemm_rows_ws_floats(B, N, K) floats);
@@ -117,9 +119,9 @@ int rows_frag_pack(const uint16_t *W, int N, int K, uint16_t *Wf, hipStream_t st
 size_t gemm_rows_ws_floats(int B, int N, int K);
 int gemm_rows(int B, int N, int K, const float *x, long ldx, const uint16_t *Wf, float *C, long ldc,
               hipStream_t st, float *ws = nullptr, size_t ws_floats = 0, bool c_zeroed = false);
-// gemm_rows with C also written as bf16 hi (rows 0 .. B-1) and lo (rows B .. 2B-1) rows of
-// hl (row stride ldhl; hi = bf16(c), lo = bf16(c - hi), the bits of split_rows2 on C), in the
-// same launch when the product runs unsplit (otherwise split_rows2 after it, ldc = ldhl = N).
+// gemm_rows with C also written as bf16 hi (rows 0 .. B-1), mid (B .. 2B-1) and lo (2B .. 3B-1)
+// rows of hl (row stride ldhl; the bits of split_rows3 on C), in the same launch when the
+// product runs unsplit (otherwise split_rows3 after it, ldc = ldhl = N).
 // xw != nullptr (unsplit products only, gemm_rows_splits(N, K) == 1): the x rows are
 // RMS-normalised with weight xw and eps xeps on the way in (the rmsnorm of k3_ops.c:94-102).
 int gemm_rows_hl(int B, int N, int K, const float *x, long ldx, const uint16_t *Wf, float *C, long ldc,
@@ -145,26 +147,22 @@ int gemm_rows_with_part(int B, int K, const float *x, long ldx, int N1, const ui
                         size_t ws_floats = 0);
 
 // Attention of an absorbed MLA decode step (kda_mla_attn.hip) in one pass over the cache:
-// the query rows qcat[b][h] = [A2[b][h] + A2[B+b][h] | q_rope(b, h)] are formed in the kernel
-// from the absorb GEMM's hi/lo halves A2 [2B][H CW] (first KL of each head's CW columns) and
+// the query rows qcat[b][h] = [sum over `planes` p of A2[pB+b][h] | q_rope(b, h)] are formed in
+// the kernel from the absorb product A2 [planes B][H CW] (first KL of each head's CW columns) and
 // q [B][H][QN + CW - KL] (rope at column QN); cache [B][cap][CW] fp32 (latent = channels
 // 0..KL-1), positions 0..Tn-1; chat = softmax(scale qcat . cache^T) . latent (its position
-// ranges merged into the bf16 hi / lo rows of ch2 [2B][H KL], 16-byte aligned), then
+// ranges merged into the bf16 hi / mid / lo rows of ch3 [3B][H KL], 16-byte aligned), then
 // o [B][H VH] = (chat_h . W_UV_h^T) * sigmoid(g) with W_UV_h the rows
 // h (QN + VH) + QN .. + VH of kvb [H (QN + VH)][KL] (bf16) and g (may be nullptr) the gate
 // logits at row stride ldg; zout[0 .. zn) = 0 on the way (may be nullptr). Shapes:
-// mla_attention_supported (H <= 64, KL a multiple of 16 up to 512, CW a multiple of 4 up to
+// mla_attention_supported (KL a multiple of 16 up to 512, CW a multiple of 4 up to
 // 576), QN % 4 == 0, KL % 8 == 0, VH <= 128. ws: mla_attention_ws_bytes bytes, 256-byte aligned; A2, q,
 // cache and kvb 16-byte aligned.
 bool mla_attention_supported(int H, int KL, int CW);
 size_t mla_attention_ws_bytes(int B, int H, int KL, int Tn);
-// lat != nullptr: position Tn - 1's cache row is written first from row b of lat (stride
-// ldlat): the first KL floats rmsnorm'd with weight lat_w and eps lat_eps, the rope slot
-// copied (the norm launch before the attention otherwise writes it).
-int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, const float *q,
-                  int QN, float *cache, const float *lat, long ldlat, const float *lat_w, float lat_eps,
-                  const uint16_t *kvb, int VH, const float *g, long ldg, float *o, float *zout, size_t zn,
-                  uint16_t *ch2, void *ws, size_t ws_bytes, hipStream_t st);
+int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, int planes, const float *q,
+                  int QN, const float *cache, const uint16_t *kvb, int VH, const float *g, long ldg, float *o, float *zout, size_t zn,
+                  uint16_t *ch3, void *ws, size_t ws_bytes, hipStream_t st);
 
 // One decode token of a KDA layer between its projections (kda_step.hip): K1 + K3 + K4 per
 // (head, sequence). Cin rows (stride ldc) hold q | k | v at columns 0, P, 2P and the beta

@@ -644,6 +644,17 @@ __global__ void split_rows2_kernel(const float *__restrict__ x, uint16_t *__rest
     }
 }
 
+__global__ void split_rows3_kernel(const float *__restrict__ x, uint16_t *__restrict__ y, size_t BN)
+{
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < BN;
+         i += (size_t)gridDim.x * blockDim.x) {
+        uint16_t p[3];
+        split3(x[i], p);
+#pragma unroll
+        for (int k = 0; k < 3; k++) y[k * BN + i] = p[k];
+    }
+}
+
 __global__ void pair_add_kernel(const float *__restrict__ C2, float *__restrict__ y, size_t BN)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < BN;
@@ -657,6 +668,15 @@ int split_rows2(const float *x, uint16_t *y, int B, int N, hipStream_t st)
     const size_t n = (size_t)B * N;
     if (!n) return K3HIP_OK;
     hipLaunchKernelGGL(split_rows2_kernel, dim3(grid_for(n)), dim3(256), 0, st, x, y, n);
+    K3_LAUNCHED();
+    return K3HIP_OK;
+}
+
+int split_rows3(const float *x, uint16_t *y, int B, int N, hipStream_t st)
+{
+    const size_t n = (size_t)B * N;
+    if (!n) return K3HIP_OK;
+    hipLaunchKernelGGL(split_rows3_kernel, dim3(grid_for(n)), dim3(256), 0, st, x, y, n);
     K3_LAUNCHED();
     return K3HIP_OK;
 }

@@ -13,16 +13,16 @@
 //
 // One decode step for B sequences that each hold `pos` cached positions: the new token's
 // latent goes to position pos and attends over 0..pos. The dense projections run on the
-// few-rows bf16 GEMM of kda_rows.hip (fp32 activations split into bf16 hi + lo in registers,
+// few-rows bf16 GEMM of kda_rows.hip (fp32 activations split into bf16 parts in registers,
 // each weight read once for all B; q_a, kv_a and g in one pass over their concatenated
 // weights), so activations keep fp32 accuracy. The absorption (W_UK_h^T q) is a bf16 MFMA
-// product per head on q's hi/lo row pairs (2B rows) against a transposed copy of W_UK made at
+// product per head on q's three split rows against a transposed copy of W_UK made at
 // upload (mla_absorb_kernel, 5.5 us at 64 heads, B = 16, against 6.2 us for the library's
 // batched GEMM: 8.4 MB of W_UK read cold each step); the final W_UV_h is applied after the
 // attention the same way. The attention reads
 // the cache once where the shape fits the fused kernel (kda_mla_attn.hip: split-bf16 MFMA
 // scores, online softmax with the reference's scale (nope+rope)^-0.5, split-bf16 weighted
-// sum of the latents; heads <= 64, kv_lora <= 512, kv_lora + rope <= 576); other shapes take
+// sum of the latents; kv_lora <= 512, kv_lora + rope <= 576); other shapes take
 // two strided-batched fp32 GEMMs (scores, then P . cache) around the reference's softmax
 // (fp32 scores times (nope+rope)^-0.5, max, expf, double sum).
 #include <math.h>
@@ -85,13 +85,29 @@ __global__ void mla_ukt_kernel(const uint16_t *__restrict__ kvb, uint16_t *__res
     }
 }
 
-// The absorb product A2[r][h][c] = sum_k x[r][h QH + k] W_UK_h[k][c] for the M = 2B rows of
-// x (q's bf16 hi rows, then its lo rows; row stride ldx) and every head h: one 16 x 16 x 32
-// bf16 MFMA tile chain per wave (16 latent columns of one head, the M rows in tiles of 16,
-// K-steps of 32 in order), fp32 results at A2 + r ldc + h CW + c. Workgroup (x, h) takes
+// The new position's latent row, written beside the absorb product (before the attention
+// reads the cache): row b of src (stride ld), the first KL floats rmsnorm'd (weight w, double
+// mean of squares, src/core/k3_ops.c:94-102), the rope slot copied, to cache row b at pos.
+// src == nullptr: the row is already there.
+struct LatRow {
+    const float *src;
+    long ld;
+    const float *w;
+    float eps;
+    float *cache;
+    long cap;
+    int pos, B;
+};
+
+// The absorb product A2[r][h][c] = sum_k x[r][h QH + k] W_UK_h[k][c] for the M = B rows of
+// x, given as bf16 hi, mid and lo planes of M rows (row stride ldx) that add up to all 24
+// bits, and every head h: one 16 x 16 x 32 bf16 MFMA tile chain per wave (16 latent columns of
+// one head, the M rows in tiles of 16, lo to hi, K-steps of 32 in order), fp32 results at
+// A2 + r ldc + h CW + c. Workgroup (x, h) takes
 // columns 64 x .. 64 x + 63 of head h. VEC: x's rows and head offsets are 16-byte aligned
 // and QN is a multiple of 8 (QH, QN and ldx multiples of 8), so each lane's 8 K values are
-// one load or none. KS = QNP / 32 K-steps, a template constant so that a tile's loads are
+// one load or none. Workgroups (x, y) with y >= H write one latent row each.
+// KS = QNP / 32 K-steps, a template constant so that a tile's loads are
 // issued together and waited for once (with a run-time count each load waited alone: 5.9 us).
 typedef __bf16 mla_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mla_f32x4 __attribute__((ext_vector_type(4)));
@@ -99,8 +115,27 @@ template <bool VEC, int KS>
 __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, int KL, int CW,
                                                          const uint16_t *__restrict__ x, long ldx,
                                                          const uint16_t *__restrict__ ukt, float *__restrict__ A2,
-                                                         long ldc)
+                                                         long ldc, int H, LatRow lr)
 {
+    if ((int)blockIdx.y >= H) {
+        __shared__ double red[16];
+        const int b = (int)(blockIdx.y - H) * gridDim.x + blockIdx.x;
+        if (b >= lr.B) return;
+        const float *src = lr.src + (size_t)b * lr.ld;
+        double ss = 0.0;
+        for (int n = threadIdx.x; n < KL; n += blockDim.x) {
+            const double v = (double)src[n];
+            ss += v * v;
+        }
+        ss = block_sum(ss, red);
+        const float inv = (float)(1.0 / sqrt(ss / (double)KL + (double)lr.eps));
+        float *dst = lr.cache + ((size_t)b * lr.cap + lr.pos) * CW;
+        for (int n = threadIdx.x; n < CW; n += blockDim.x) {
+            const float v = src[n];
+            dst[n] = n < KL ? (lr.w[n] * v) * inv : v;
+        }
+        return;
+    }
     constexpr int QNP = 32 * KS;
     const int h = blockIdx.y, lane = threadIdx.x & 63;
     const int n0 = 64 * blockIdx.x + 16 * (threadIdx.x >> 6);
@@ -114,29 +149,33 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, 
     for (int m0 = 0; m0 < M; m0 += 16) {
         const int r = m0 + (lane & 15);
         const uint16_t *xr = x + (size_t)(r < M ? r : 0) * ldx + (size_t)h * QH + kq;
-        mla_bf16x8 af[KS];
+        mla_bf16x8 af[3][KS];
 #pragma unroll
-        for (int t = 0; t < KS; t++) {
+        for (int pt = 0; pt < 3 * KS; pt++) {
+            const int p = pt / KS, t = pt % KS;
+            const uint16_t *xp = xr + (size_t)p * M * ldx;
             mla_bf16x8 a;
             if constexpr (VEC) {
                 // QN % 8 == 0: an 8-value group is wholly inside or past QN; a group past it (or
                 // a row past M) loads the head's first group instead and is zeroed, so every
                 // load is issued unconditionally from an address inside the row
                 const bool ok = r < M && 32 * t + kq < QN;
-                const mla_bf16x8 v = *reinterpret_cast<const mla_bf16x8 *>(xr + (ok ? 32 * t : -kq));
+                const mla_bf16x8 v = *reinterpret_cast<const mla_bf16x8 *>(xp + (ok ? 32 * t : -kq));
                 a = ok ? v : mla_bf16x8{};
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
                     const int k = 32 * t + kq + e;
-                    a[e] = __builtin_bit_cast(__bf16, r < M && k < QN ? xr[32 * t + e] : (uint16_t)0);
+                    a[e] = __builtin_bit_cast(__bf16, r < M && k < QN ? xp[32 * t + e] : (uint16_t)0);
                 }
             }
-            af[t] = a;
+            af[p][t] = a;
         }
         mla_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int t = 0; t < KS; t++) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[t], bf[t], c, 0, 0, 0);
+        for (int p = 2; p >= 0; p--)
+#pragma unroll
+            for (int t = 0; t < KS; t++) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], bf[t], c, 0, 0, 0);
         // C layout: lane l holds rows 4 (l / 16) + i of the tile, column l % 16
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -148,10 +187,11 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, 
 
 template <bool VEC>
 static int mla_absorb_v(int M, int H, int QH, int QN, int QNP, int KL, int CW, const uint16_t *x, long ldx,
-                        const uint16_t *ukt, float *A2, long ldc, hipStream_t st)
+                        const uint16_t *ukt, float *A2, long ldc, const LatRow &lr, hipStream_t st)
 {
-    const dim3 grid((unsigned)((KL + 63) / 64), (unsigned)H);
-#define K3_ABS(KS) hipLaunchKernelGGL((mla_absorb_kernel<VEC, KS>), grid, dim3(256), 0, st, M, QH, QN, KL, CW, x, ldx, ukt, A2, ldc)
+    const int gx = (KL + 63) / 64;
+    const dim3 grid((unsigned)gx, (unsigned)(H + (lr.src ? (lr.B + gx - 1) / gx : 0)));
+#define K3_ABS(KS) hipLaunchKernelGGL((mla_absorb_kernel<VEC, KS>), grid, dim3(256), 0, st, M, QH, QN, KL, CW, x, ldx, ukt, A2, ldc, H, lr)
     switch (QNP / 32) {
     case 1: K3_ABS(1); break;
     case 2: K3_ABS(2); break;
@@ -168,13 +208,14 @@ static int mla_absorb_v(int M, int H, int QH, int QN, int QNP, int KL, int CW, c
     return K3HIP_OK;
 }
 
-// A2 = per head h, x (M rows, columns h QH .. h QH + QN - 1) . W_UK_h, via mla_absorb_kernel.
+// A2 = per head h, x (M rows in three planes, columns h QH .. h QH + QN - 1) . W_UK_h, via
+// mla_absorb_kernel.
 static int mla_absorb(int M, int H, int QH, int QN, int QNP, int KL, int CW, const uint16_t *x, long ldx,
-                      const uint16_t *ukt, float *A2, long ldc, hipStream_t st)
+                      const uint16_t *ukt, float *A2, long ldc, const LatRow &lr, hipStream_t st)
 {
     if (QH % 8 == 0 && QN % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0)
-        return mla_absorb_v<true>(M, H, QH, QN, QNP, KL, CW, x, ldx, ukt, A2, ldc, st);
-    return mla_absorb_v<false>(M, H, QH, QN, QNP, KL, CW, x, ldx, ukt, A2, ldc, st);
+        return mla_absorb_v<true>(M, H, QH, QN, QNP, KL, CW, x, ldx, ukt, A2, ldc, lr, st);
+    return mla_absorb_v<false>(M, H, QH, QN, QNP, KL, CW, x, ldx, ukt, A2, ldc, lr, st);
 }
 
 __global__ void mla_norm_kernel(long ldc, float eps, NormJob j0, NormJob j1, long cap, int pos)
@@ -201,9 +242,9 @@ __global__ void mla_norm_kernel(long ldc, float eps, NormJob j0, NormJob j1, lon
     }
 }
 
-// qcat[b][h] = [ A2[b][h] + A2[B+b][h] (the absorbed W_UK_h^T q_nope, kv_lora floats) |
-// q_rope(b,h) ], from the hi/lo halves of the batched absorb GEMM and the fp32 q.
-__global__ void mla_qcat_kernel(const float *__restrict__ A2, const float *__restrict__ q, int B,
+// qcat[b][h] = [ sum over planes p of A2[pB+b][h] (the absorbed W_UK_h^T q_nope, kv_lora floats) |
+// q_rope(b,h) ], from the absorb product's planes and the fp32 q.
+__global__ void mla_qcat_kernel(const float *__restrict__ A2, int planes, const float *__restrict__ q, int B,
                                 int H, int QN, int QR, int KL, float *__restrict__ qcat)
 {
     const int W = KL + QR, QH = QN + QR;
@@ -212,7 +253,10 @@ __global__ void mla_qcat_kernel(const float *__restrict__ A2, const float *__res
          i += (size_t)gridDim.x * blockDim.x) {
         const size_t bh = i / W;
         const int c = (int)(i % W);
-        qcat[i] = c < KL ? A2[i] + A2[n + i] : q[bh * QH + QN + (c - KL)];
+        float v = c < KL ? A2[i] : q[bh * QH + QN + (c - KL)];
+        if (c < KL)
+            for (int p = 1; p < planes; p++) v += A2[(size_t)p * n + i];
+        qcat[i] = v;
     }
 }
 
@@ -241,7 +285,7 @@ __global__ void mla_softmax_kernel(float *__restrict__ S, int n, int ld, float s
     for (int t = threadIdx.x; t < ld; t += blockDim.x) row[t] = t < n ? (float)((double)row[t] / z) : 0.0f;
 }
 
-// o = O2[b] + O2[B+b] (the halves of the batched W_UV GEMM), times sigmoid(g) when gated
+// o = O2[b] + O2[B+b] + O2[2B+b] (the planes of the batched W_UV GEMM), times sigmoid(g) when gated
 // (g row b at stride ldg), as fp32 rows of o [B][H*VH] for o_proj; zout[0 .. zn) = 0 on the
 // way (may be nullptr) for an o_proj that adds its two K-range partials there.
 __global__ void mla_gate_kernel(const float *__restrict__ O2, const float *__restrict__ g, long ldg,
@@ -249,7 +293,7 @@ __global__ void mla_gate_kernel(const float *__restrict__ O2, const float *__res
 {
     const size_t n = (size_t)B * HV, step = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step) {
-        float v = O2[i] + O2[n + i];
+        float v = O2[i] + (O2[n + i] + O2[2 * n + i]);
         if (g) v *= 1.0f / (1.0f + expf(-g[(i / HV) * ldg + i % HV]));
         o[i] = v;
     }
@@ -436,9 +480,11 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     // attention in one pass over the cache (kda_mla_attn.hip) where the shape fits it, else
     // as two strided-batched fp32 GEMMs around the softmax
     const bool fused = mla_attention_supported(H, KL, CW) && !((uintptr_t)cache & 15) && !(QN & 3) && VH <= 128;
-    // scratch: q_a kv_a g projections [B][ld1] | q_a normed | q | q hi/lo | absorb halves | qcat |
-    //          scores or the fused attention's workspace | chat | chat hi/lo | W_UV halves (chat
-    //          and the W_UV halves only without the fused attention) | o | split-K partials
+    // planes of the absorb product: one from the absorb kernel, three from the library GEMM
+    const int planes = w->ukt ? 1 : 3;
+    // scratch: q_a kv_a g projections [B][ld1] | q_a normed | q | q split | absorb planes | qcat |
+    //          scores or the fused attention's workspace | chat | chat split | W_UV planes (qcat,
+    //          chat and the W_UV planes only without the fused attention) | o | split-K partials
     const int N1 = QL + CW + (w->gate ? HV : 0);
     const long ld1 = (N1 + 3) & ~3;
     // the q_a / kv_a / g product on K-ranges that spread it over every CU, summed by a second
@@ -447,10 +493,11 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     const size_t wsf = std::max({gemm_rows_ws_floats(B, N1, E), np1 > 1 ? (size_t)np1 * std::min(64, B) * N1 : 0,
                                  gemm_rows_ws_floats(B, H * QH, QL), gemm_rows_ws_floats(B, E, HV)});
     size_t sizes[] = {(size_t)B * ld1 * 4, (size_t)B * QL * 4, (size_t)B * H * QH * 4,
-                      (size_t)2 * B * H * QH * 2, (size_t)2 * B * H * CW * 4, (size_t)B * H * CW * 4,
+                      (size_t)3 * B * H * QH * 2, (size_t)planes * B * H * CW * 4,
+                      fused ? 0 : (size_t)B * H * CW * 4,
                       fused ? mla_attention_ws_bytes(B, H, KL, Tn) : (size_t)B * H * Tn * 4,
-                      fused ? 0 : (size_t)B * H * KL * 4, (size_t)2 * B * H * KL * 2,
-                      fused ? 0 : (size_t)2 * B * HV * 4, (size_t)B * HV * 4, wsf * 4};
+                      fused ? 0 : (size_t)B * H * KL * 4, (size_t)3 * B * H * KL * 2,
+                      fused ? 0 : (size_t)3 * B * HV * 4, (size_t)B * HV * 4, wsf * 4};
     constexpr int NB = sizeof sizes / sizeof sizes[0];
     size_t off[NB], total = 0;
     for (int i = 0; i < NB; i++) {
@@ -462,45 +509,47 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     if (rc) return rc;
     char *base = (char *)buf.p;
     float *C1 = (float *)(base + off[0]), *qn = (float *)(base + off[1]), *q = (float *)(base + off[2]);
-    uint16_t *qs2 = (uint16_t *)(base + off[3]);
+    uint16_t *qs3 = (uint16_t *)(base + off[3]);
     float *A2 = (float *)(base + off[4]), *qcat = (float *)(base + off[5]), *S = (float *)(base + off[6]);
     float *chat = (float *)(base + off[7]);
-    uint16_t *ch2 = (uint16_t *)(base + off[8]);
+    uint16_t *ch3 = (uint16_t *)(base + off[8]);
     float *O2 = (float *)(base + off[9]), *o = (float *)(base + off[10]), *ws = (float *)(base + off[11]);
     const uint16_t *kvb = (const uint16_t *)w->kv_b;
 
-    // q_a, kv_a and g in one pass over their weights (fp32 x split hi/lo in registers);
+    // q_a, kv_a and g in one pass over their weights (fp32 x split in registers);
     // q = q_b(rmsnorm(q_a x)); latent + rope = kv_a x, the latent rmsnorm'd into the cache
     if ((rc = gemm_rows_even(B, N1, E, x, E, (const uint16_t *)w->xin, C1, ld1, st, ws, wsf))) return rc;
-    // the two rmsnorms: with the fused attention and an unsplit q_b product, the q_b GEMV
-    // normalises q_a as it reads it and the attention writes the new latent row itself;
+    // the two rmsnorms: with the absorb kernel and an unsplit q_b product, the q_b GEMV
+    // normalises q_a as it reads it and the absorb launch writes the new latent row;
     // otherwise one launch writes qn and the cache row
-    const bool fold_norms = fused && gemm_rows_splits(H * QH, QL) == 1 && !((uintptr_t)w->q_a_norm & 15);
+    const bool fold_norms = fused && w->ukt && gemm_rows_splits(H * QH, QL) == 1 && !((uintptr_t)w->q_a_norm & 15);
     if (!fold_norms) {
         hipLaunchKernelGGL(mla_norm_kernel, dim3(B, 2), dim3(256), 0, st, ld1, w->eps,
                            NormJob{C1, QL, QL, w->q_a_norm, qn, nullptr},
                            NormJob{C1 + QL, CW, KL, w->kv_a_norm, nullptr, cache}, (long)cap, pos);
         K3_LAUNCHED();
     }
-    // q, and q as bf16 hi / lo rows for the absorb GEMM, from one launch
+    // q, and q as bf16 hi / mid / lo rows for the absorb product, from one launch
     if (fold_norms)
-        rc = gemm_rows_hl(B, H * QH, QL, C1, ld1, (const uint16_t *)w->q_b, q, (long)H * QH, qs2, (long)H * QH, st, ws,
+        rc = gemm_rows_hl(B, H * QH, QL, C1, ld1, (const uint16_t *)w->q_b, q, (long)H * QH, qs3, (long)H * QH, st, ws,
                           wsf, w->q_a_norm, w->eps);
     else
-        rc = gemm_rows_hl(B, H * QH, QL, qn, QL, (const uint16_t *)w->q_b, q, (long)H * QH, qs2, (long)H * QH, st, ws,
+        rc = gemm_rows_hl(B, H * QH, QL, qn, QL, (const uint16_t *)w->q_b, q, (long)H * QH, qs3, (long)H * QH, st, ws,
                           wsf);
     if (rc) return rc;
-    // absorb: per head h, [q hi; lo] (2B x QN) . W_UK_h (QN x KL)
+    // absorb: per head h, [q hi; mid; lo] (3B x QN) . W_UK_h (QN x KL)
     if (w->ukt) {
-        if ((rc = mla_absorb(2 * B, H, QH, QN, w->QNP, KL, CW, qs2, (long)H * QH, (const uint16_t *)w->ukt, A2,
-                             (long)H * CW, st)))
+        if ((rc = mla_absorb(B, H, QH, QN, w->QNP, KL, CW, qs3, (long)H * QH, (const uint16_t *)w->ukt, A2,
+                             (long)H * CW,
+                             LatRow{fold_norms ? C1 + QL : nullptr, ld1, w->kv_a_norm, w->eps, cache, (long)cap, pos, B},
+                             st)))
             return rc;
     } else {
         GemmDesc ga;
-        ga.M = 2 * B; ga.N = KL; ga.K = QN; ga.ab_dtype = K3HIP_BF16; ga.c_dtype = K3HIP_F32; ga.b_trans = false;
+        ga.M = 3 * B; ga.N = KL; ga.K = QN; ga.ab_dtype = K3HIP_BF16; ga.c_dtype = K3HIP_F32; ga.b_trans = false;
         ga.lda = (long)H * QH; ga.ldb = KL; ga.ldc = (long)H * CW; ga.batch = H;
         ga.sa = QH; ga.sb = (long)(QN + VH) * KL; ga.sc = CW;
-        if ((rc = gemm(ga, qs2, kvb, A2, st))) return rc;
+        if ((rc = gemm(ga, qs3, kvb, A2, st))) return rc;
     }
     // o_proj as two K-ranges adds into `out`, zeroed by the kernel before it (no reduction
     // launch); atomics on ordinary device memory only
@@ -509,16 +558,15 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     if (fused) {
         // the query rows formed inside the attention from A2 and q; the ranges merged, W_UV and
         // the output gate applied in the launch after it (kda_mla_attn.hip)
-        if ((rc = mla_attention(B, H, KL, CW, Tn, cap, 1.0f / sqrtf((float)QH), A2, q, QN, cache,
-                                fold_norms ? C1 + QL : nullptr, ld1, w->kv_a_norm, w->eps, kvb, VH, gl, ld1,
-                                o, oz ? out : nullptr, oz ? (size_t)B * E : (size_t)0, ch2, S,
+        if ((rc = mla_attention(B, H, KL, CW, Tn, cap, 1.0f / sqrtf((float)QH), A2, planes, q, QN, cache, kvb, VH, gl, ld1,
+                                o, oz ? out : nullptr, oz ? (size_t)B * E : (size_t)0, ch3, S,
                                 mla_attention_ws_bytes(B, H, KL, Tn), st)))
             return rc;
         return gemm_rows(B, E, HV, o, HV, (const uint16_t *)w->o, out, E, st, ws, wsf, oz);
     }
     {
-        hipLaunchKernelGGL(mla_qcat_kernel, dim3(mla_grid((size_t)B * H * CW)), dim3(256), 0, st, A2, q, B, H,
-                           QN, QR, KL, qcat);
+        hipLaunchKernelGGL(mla_qcat_kernel, dim3(mla_grid((size_t)B * H * CW)), dim3(256), 0, st, A2, planes, q,
+                           B, H, QN, QR, KL, qcat);
         K3_LAUNCHED();
         // scores S_b [H][Tn] = qcat_b [H][CW] . cache_b[0..Tn)^T, per sequence
         GemmDesc gs;
@@ -544,14 +592,14 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
         gp.sa = (long)H * Tn; gp.sb = (long)cap * CW; gp.sc = (long)H * KL;
         gp.cache = false;
         if ((rc = gemm(gp, S, cache, chat, st))) return rc;
-        if ((rc = split_rows2(chat, ch2, B, H * KL, st))) return rc;
+        if ((rc = split_rows3(chat, ch3, B, H * KL, st))) return rc;
     }
-    // W_UV: per head h, [chat hi; lo] (2B x KL) . W_UV_h^T (KL x VH), batched over heads; gate
+    // W_UV: per head h, [chat hi; mid; lo] (3B x KL) . W_UV_h^T (KL x VH), batched over heads; gate
     GemmDesc gu;
-    gu.M = 2 * B; gu.N = VH; gu.K = KL; gu.ab_dtype = K3HIP_BF16; gu.c_dtype = K3HIP_F32; gu.b_trans = true;
+    gu.M = 3 * B; gu.N = VH; gu.K = KL; gu.ab_dtype = K3HIP_BF16; gu.c_dtype = K3HIP_F32; gu.b_trans = true;
     gu.lda = (long)H * KL; gu.ldb = KL; gu.ldc = HV; gu.batch = H;
     gu.sa = KL; gu.sb = (long)(QN + VH) * KL; gu.sc = VH;
-    if ((rc = gemm(gu, ch2, kvb + (size_t)QN * KL, O2, st))) return rc;
+    if ((rc = gemm(gu, ch3, kvb + (size_t)QN * KL, O2, st))) return rc;
     hipLaunchKernelGGL(mla_gate_kernel, dim3(mla_grid((size_t)B * HV)), dim3(256), 0, st, O2, gl, ld1, B,
                        (size_t)HV, o, oz ? out : nullptr, oz ? (size_t)B * E : (size_t)0);
     K3_LAUNCHED();

@@ -10,8 +10,10 @@
 // kv_b absorbed. The cache (302 MB at 16 sequences x 8192 positions x 576 floats) dominates
 // the bytes, so the kernel reads it exactly once, and everything else stays on the chip:
 //
-//  * A workgroup (8 waves, two per SIMD) owns one sequence and a contiguous range of
-//    positions (~CUs/B ranges per sequence) and walks it in tiles of 16 positions (16
+//  * A workgroup (8 waves, two per SIMD) owns one sequence, up to 64 heads (more heads are
+//    dealt evenly over groups, which find the cache rows in L2 and the memory-side cache)
+//    and a contiguous range of positions (CUs / (B groups) ranges, rounded down so that one
+//    round of workgroups covers the GPU) and walks it in tiles of 16 positions (16
 //    contiguous cache rows). Every thread loads its 16-byte units of a tile one iteration
 //    ahead into registers, splits them into bf16 hi/lo and stages them row-major in LDS
 //    (four tile buffers: the tile being scored, the two being summed, the next one).
@@ -34,7 +36,7 @@
 //    One barrier per iteration: P of tile it and the staging of tile it + 1 are published.
 //  * Each workgroup writes its unnormalised sums with (M, l); a second kernel merges the
 //    ranges of a sequence (weights 2^(M_s - M*), the sums in a fixed order), divides by the
-//    merged sum and writes chat directly as the bf16 hi/lo rows of the W_UV GEMM.
+//    merged sum and writes chat directly as the bf16 hi/mid/lo rows of the W_UV product.
 #include <math.h>
 
 #include <algorithm>
@@ -79,28 +81,17 @@ constexpr size_t AT_P = (size_t)AT_NB * 2 * AT_PLANE * 2;  // bytes: tiles; then
 constexpr size_t AT_A = AT_P + 2 * 4 * 64 * 16;              // rescale factors [2][4][64] fp32
 constexpr size_t AT_LDS = AT_A + 2 * 4 * 64 * 4;
 
+// H heads in groups of HG (a multiple of 16, at most 64; the last may hold fewer)
 struct AtGeom {
-    int H, CW, KL;
+    int H, HG, CW, KL;
 };
 
-// Where the query rows come from: qcat[b][h] = [A2[b][h] + A2[B+b][h] (the hi and lo halves
-// of the batched absorb GEMM, KL floats) | q_rope(b, h) (q [B][H][QH] at column QN)], formed
-// while the q fragments are loaded (the same fp32 sums a separate qcat pass would store).
+// Where the query rows come from: qcat[b][h] = [sum over planes p of A2[pB+b][h] (one plane from
+// the absorb kernel, three from the batched library GEMM on q's split rows; KL floats) |
+// q_rope(b, h) (q [B][H][QH] at column QN)], formed while the q fragments are loaded.
 struct AtQ {
     const float *A2, *q;
-    int B, QN, QH;
-};
-
-// The new position's cache row, written by the workgroup that owns the last range before it
-// reads any cache row: the rmsnorm'd latent (weight w, double mean of squares,
-// src/core/k3_ops.c:94-102) and the rope slot copied, from row b of src (stride ld). src ==
-// nullptr: the row is already in the cache.
-struct AtRow {
-    const float *src;
-    long ld;
-    const float *w;
-    float eps;
-    int pos;
+    int planes, B, QN, QH;
 };
 
 __device__ __forceinline__ void split2(float a, float b, bf16x2 &hi, bf16x2 &lo)
@@ -110,15 +101,22 @@ __device__ __forceinline__ void split2(float a, float b, bf16x2 &hi, bf16x2 &lo)
     lo = __builtin_convertvector(f2{a - __uint_as_float(u << 16), b - __uint_as_float(u & 0xffff0000u)}, bf16x2);
 }
 
-// Workgroup (sp, b): positions [Tn sp / nsplit, Tn (sp + 1) / nsplit) of sequence b.
+// Workgroup (sp, b, z): positions [Tn sp / nsplit, Tn (sp + 1) / nsplit) of sequence b, heads
+// z HG .. of the group (h and H below count within it; h0 is its first). NHT: 16-head tiles
+// of a group, so that groups of fewer than 64 heads spend no products on absent ones (16 heads,
+// 16 sequences x 8192 positions, hidden 4096: the layer 118.7 -> 111.6 us). LL: the weighted sum
+// also takes the lo x lo products, for head counts beyond 64: two fp32 GEMMs around a softmax
+// served those before (96 heads, 3 sequences x 3001 positions: the layer 156.5 -> 127 us, 16
+// x 8192: 383 -> 219 us), and without them the layer's error against 64 bits was up to 15%
+// above theirs on short contexts.
 // Wave w: S role for w < 4 (head tile ht = w: heads 16 ht .. 16 ht + 15; lane l works for
 // head h = 16 ht + (l & 15), kg = l >> 4 picks its K slice in the score product and its 4
 // positions of each tile, 4 kg .. 4 kg + 3), U role otherwise (latent channel quarter
 // w - 4, all head tiles). FULL: kv_lora + rope = 576, every staging unit of a row exists.
-template <bool FULL>
+template <bool FULL, int NHT, bool LL>
 __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void mla_attn_kernel(
-    AtGeom g, int Tn, int cap, int nsplit, float scale2, AtQ qs, AtRow nr,
-    float *__restrict__ cache, float *__restrict__ pctx, float *__restrict__ pm, float *__restrict__ pl)
+    AtGeom g, int Tn, int cap, int nsplit, float scale2, AtQ qs,
+    const float *__restrict__ cache, float *__restrict__ pctx, float *__restrict__ pm, float *__restrict__ pl)
 {
     extern __shared__ __attribute__((aligned(16))) uint16_t at_smem[];
     char *sbase = reinterpret_cast<char *>(at_smem);
@@ -128,7 +126,8 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     const int sp = blockIdx.x, b = blockIdx.y;
     const int p0 = (int)((long)Tn * sp / nsplit), p1 = (int)((long)Tn * (sp + 1) / nsplit);
     const int ntile = (p1 - p0 + AT_T - 1) / AT_T;
-    const int H = g.H, CW = FULL ? 32 * AT_MAXKS : g.CW, KL = g.KL;
+    const int Hall = g.H, h0 = (int)blockIdx.z * g.HG, H = min(g.HG, Hall - h0);
+    const int CW = FULL ? 32 * AT_MAXKS : g.CW, KL = g.KL;
     const int h = 16 * ht + m;
     const bool act = 16 * ht < H;   // wave-uniform: this wave has heads
 
@@ -165,37 +164,7 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
             }
     };
 
-    // the workgroup of the last range writes the new position's row (Tn - 1 = pos) first;
-    // tile 0 goes out before that unless it is the tile that holds the row
-    const bool own_row = nr.src && sp == nsplit - 1;
-    if (!own_row || ntile > 1) load_tile(0);
-    if (own_row) {
-        const float *src = nr.src + (size_t)b * nr.ld;
-        double ss = 0.0;
-        for (int n = tid; n < KL; n += AT_NT) {
-            const double v = (double)src[n];
-            ss += v * v;
-        }
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
-        double *red = reinterpret_cast<double *>(at_smem);
-        if (lane == 0) red[w] = ss;
-        __syncthreads();
-        ss = 0.0;
-#pragma unroll
-        for (int i = 0; i < AT_NT / 64; i++) ss += red[i];
-        const float inv = (float)(1.0 / sqrt(ss / (double)KL + (double)nr.eps));
-        float *dst = cache + ((size_t)b * cap + nr.pos) * CW;
-        for (int n = tid; n < CW; n += AT_NT) {
-            const float v = src[n];
-            dst[n] = n < KL ? (nr.w[n] * v) * inv : v;
-        }
-        // the row is read back only by this workgroup's own cache loads (which go to L2: no
-        // line of it was loaded here before): its stores complete, then every wave goes on
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        __syncthreads();
-    }
-    if (own_row && ntile <= 1) load_tile(0);
+    load_tile(0);
     stage(0);
     load_tile(1);
     __syncthreads();
@@ -214,16 +183,19 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
                 float x[8];
                 const int c = 32 * i + 8 * kg;
                 const bool ok = h < H;
-                const size_t bh = (size_t)b * H + (ok ? h : 0);
-                const float *a2 = qs.A2 + bh * CW, *a2lo = a2 + (size_t)qs.B * H * CW;
+                const size_t bh = (size_t)b * Hall + h0 + (ok ? h : 0);
+                const float *a2 = qs.A2 + bh * CW;
                 const float *qr = qs.q + bh * qs.QH + qs.QN - KL;
 #pragma unroll
                 for (int e = 0; e < 8; e += 4) {
                     const int cc = c + e;
                     f4 v = f4{0.0f, 0.0f, 0.0f, 0.0f};
                     if (ok && cc < CW) {
-                        if (cc < KL) v = *reinterpret_cast<const f4 *>(a2 + cc) + *reinterpret_cast<const f4 *>(a2lo + cc);
-                        else v = *reinterpret_cast<const f4 *>(qr + cc);
+                        if (cc < KL) {
+                            v = *reinterpret_cast<const f4 *>(a2 + cc);
+                            for (int p = 1; p < qs.planes; p++)
+                                v += *reinterpret_cast<const f4 *>(a2 + (size_t)p * qs.B * Hall * CW + cc);
+                        } else v = *reinterpret_cast<const f4 *>(qr + cc);
                     }
                     x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
                 }
@@ -320,28 +292,28 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         lsum += __shfl_xor(lsum, 16, 64);
         lsum += __shfl_xor(lsum, 32, 64);
         if (act && h < H && kg == 0) {
-            pm[((size_t)b * nsplit + sp) * H + h] = M;
-            pl[((size_t)b * nsplit + sp) * H + h] = lsum;
+            pm[((size_t)b * nsplit + sp) * Hall + h0 + h] = M;
+            pl[((size_t)b * nsplit + sp) * Hall + h0 + h] = lsum;
         }
     } else {
-        // U wave u = w - 4 owns latent channel tiles 8 u .. 8 u + 7 for all four head tiles:
+        // U wave u = w - 4 owns latent channel tiles 8 u .. 8 u + 7 for all head tiles:
         // acc[jj][g] = chat^T[channel 16 (8 u + jj) + 4 kg + e][head 16 g + m], so each latent
         // fragment is read from LDS by one wave only (a wave per head tile would read every
         // fragment four times and make the LDS the bound)
         const int u = w - 4;
-        f32x4 acc[AT_UCT][4];
+        f32x4 acc[AT_UCT][NHT];
 #pragma unroll
         for (int jj = 0; jj < AT_UCT; jj++)
 #pragma unroll
-            for (int g2 = 0; g2 < 4; g2++) acc[jj][g2] = 0.0f;
+            for (int g2 = 0; g2 < NHT; g2++) acc[jj][g2] = 0.0f;
         // P operands per head tile g2. Lane (head 16 g2 + m, K slice kg) supplies positions
         // 4 (kg & 1) .. + 3 and 8 + 4 (kg & 1) .. + 3 of the pair's tile kg >> 1 (so that each
         // 32-lane half of a transposed read covers 8 rows of one half of the tile, on distinct
         // banks): the entries (hi01, hi23, lo01, lo23) of the head's S lanes kg & 1 and
         // 2 + (kg & 1). The lanes of the pair's first tile (kg < 2) read theirs one iteration
         // early: the S waves overwrite that P buffer in the pair's iteration.
-        uint4 pa[4], pb[4];
-        float al0[4];
+        uint4 pa[NHT], pb[NHT];
+        float al0[NHT];
         const int src0 = m + 16 * (kg & 1), src1 = src0 + 32;
         auto p_entry = [&](int t, int g2, int src) {
             return *reinterpret_cast<const uint4 *>(sbase + AT_P + ((size_t)((t & 1) * 4 + g2) * 64 + src) * 16);
@@ -351,16 +323,16 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         };
         auto u_grab = [&](int t0) {
             // every read first, one wait
-            float a[4];
-            uint4 xa[4], xb[4];
+            float a[NHT];
+            uint4 xa[NHT], xb[NHT];
 #pragma unroll
-            for (int g2 = 0; g2 < 4; g2++) {
+            for (int g2 = 0; g2 < NHT; g2++) {
                 a[g2] = alpha_of(t0, g2);
                 xa[g2] = p_entry(t0, g2, src0);
                 xb[g2] = p_entry(t0, g2, src1);
             }
 #pragma unroll
-            for (int g2 = 0; g2 < 4; g2++) {
+            for (int g2 = 0; g2 < NHT; g2++) {
                 const bool hg = 16 * g2 < H;   // head tiles without heads: weight zero
                 al0[g2] = hg ? a[g2] : 1.0f;
                 if (!(kg >> 1)) {
@@ -373,17 +345,17 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         auto u_pair = [&](int t0) {
             const int t1 = t0 + 1;
             const bool has1 = t1 < ntile;
-            float a[4];
-            uint4 xa[4], xb[4];
+            float a[NHT];
+            uint4 xa[NHT], xb[NHT];
 #pragma unroll
-            for (int g2 = 0; g2 < 4; g2++) {
+            for (int g2 = 0; g2 < NHT; g2++) {
                 a[g2] = alpha_of(t1, g2);
                 xa[g2] = p_entry(t1, g2, src0);
                 xb[g2] = p_entry(t1, g2, src1);
             }
-            bf16x8 ph[4], pq[4];
+            bf16x8 ph[NHT], pq[NHT];
 #pragma unroll
-            for (int g2 = 0; g2 < 4; g2++) {
+            for (int g2 = 0; g2 < NHT; g2++) {
                 const bool hg = 16 * g2 < H, use1 = has1 && hg;
                 const float al1 = use1 ? a[g2] : 1.0f;
                 if (kg >> 1) {
@@ -425,8 +397,8 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
                 return __builtin_bit_cast(bf16x8, uint4{__builtin_bit_cast(uint2, x0).x, __builtin_bit_cast(uint2, x0).y,
                                                         __builtin_bit_cast(uint2, x1).x, __builtin_bit_cast(uint2, x1).y});
             };
-            // per channel tile: each of the three split products over the four head tiles (four
-            // independent chains hide the ~40-cycle latency of a dependent MFMA); the latent
+            // per channel tile: each of the three split products over the head tiles (four
+            // independent chains at 64 heads hide the ~40-cycle latency of a dependent MFMA); the latent
             // fragments are read AT_UPF channel tiles ahead
             bf16x8 rh[AT_UPF], rl[AT_UPF];
 #pragma unroll
@@ -439,13 +411,18 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
             for (int jj = 0; jj < AT_UCT; jj++) {
                 const bf16x8 ah = rh[jj % AT_UPF], al = rl[jj % AT_UPF];
 #pragma unroll
-                for (int g2 = 0; g2 < 4; g2++)
+                for (int g2 = 0; g2 < NHT; g2++)
                     acc[jj][g2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, ph[g2], acc[jj][g2], 0, 0, 0);
+                if constexpr (LL) {
 #pragma unroll
-                for (int g2 = 0; g2 < 4; g2++)
+                    for (int g2 = 0; g2 < NHT; g2++)
+                        acc[jj][g2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, pq[g2], acc[jj][g2], 0, 0, 0);
+                }
+#pragma unroll
+                for (int g2 = 0; g2 < NHT; g2++)
                     acc[jj][g2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, pq[g2], acc[jj][g2], 0, 0, 0);
 #pragma unroll
-                for (int g2 = 0; g2 < 4; g2++)
+                for (int g2 = 0; g2 < NHT; g2++)
                     acc[jj][g2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, ph[g2], acc[jj][g2], 0, 0, 0);
                 if (jj + AT_UPF < AT_UCT) {
                     rl[jj % AT_UPF] = rd(lo, jj + AT_UPF);
@@ -464,10 +441,10 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         }
         if (uact) {
 #pragma unroll
-            for (int g2 = 0; g2 < 4; g2++) {
+            for (int g2 = 0; g2 < NHT; g2++) {
                 const int hh = 16 * g2 + m;
                 if (hh >= H) continue;
-                float *outp = pctx + (((size_t)b * nsplit + sp) * H + hh) * KL + 4 * kg;
+                float *outp = pctx + (((size_t)b * nsplit + sp) * Hall + h0 + hh) * KL + 4 * kg;
 #pragma unroll
                 for (int jj = 0; jj < AT_UCT; jj++) {
                     const int j = AT_UCT * u + jj;
@@ -480,13 +457,13 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 }
 
 // Block (h, b): merge the nsplit ranges of sequence b, head h, in range order; write
-// chat = sum / l as bf16 hi (row b) and lo (row B + b) of ch2 [2B][H KL]. Thread i covers
+// chat = sum / l as bf16 hi (row b), mid (row B + b) and lo (row 2B + b) of ch3 [3B][H KL]. Thread i covers
 // channels 4i .. 4i + 3 (and every 4 * blockDim further).
 __global__ __launch_bounds__(128) void mla_attn_merge_kernel(int B, int H, int KL, int nsplit,
                                                              const float *__restrict__ pctx,
                                                              const float *__restrict__ pm,
                                                              const float *__restrict__ pl,
-                                                             uint16_t *__restrict__ ch2)
+                                                             uint16_t *__restrict__ ch3)
 {
     __shared__ float sw[AT_MAXSPLIT];
     __shared__ float sl;
@@ -517,19 +494,18 @@ __global__ __launch_bounds__(128) void mla_attn_merge_kernel(int B, int H, int K
             a += sw[s] * *reinterpret_cast<const f4 *>(pctx + (((size_t)b * nsplit + s) * H + h) * KL + c);
         const size_t i = ((size_t)b * H + h) * KL + c;
         const float v[4] = {a.x * rl, a.y * rl, a.z * rl, a.w * rl};
-        uint16_t hv[4], lv[4];
+        uint16_t p[4][3];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            hv[e] = f2bf(v[e]);
-            lv[e] = f2bf(v[e] - bf2f(hv[e]));
-        }
-        *reinterpret_cast<uint2 *>(ch2 + i) = uint2{hv[0] | ((uint32_t)hv[1] << 16), hv[2] | ((uint32_t)hv[3] << 16)};
-        *reinterpret_cast<uint2 *>(ch2 + BN + i) = uint2{lv[0] | ((uint32_t)lv[1] << 16), lv[2] | ((uint32_t)lv[3] << 16)};
+        for (int e = 0; e < 4; e++) split3(v[e], p[e]);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            *reinterpret_cast<uint2 *>(ch3 + k * BN + i) =
+                uint2{p[0][k] | ((uint32_t)p[1][k] << 16), p[2][k] | ((uint32_t)p[3][k] << 16)};
     }
 }
 
 // o = (chat . W_UV_h^T) * sigmoid(g) per (head h, block of up to 16 sequences) from the merged
-// chat's bf16 hi / lo rows (ch2 [2B][H KL]): both halves against the bf16 weight into one fp32
+// chat's bf16 hi / mid / lo rows (ch3 [3B][H KL]): all three against the bf16 weight into one fp32
 // accumulator on 16x16x32 MFMA (the products exact, the sums fp32), then the output gate
 // sigmoid(g) (the reference's 1 / (1 + expf(-g)), src/core/k3_ops.c:105), written as fp32
 // rows of o [B][H VH] for o_proj. Replaces a head-batched W_UV GEMM and a gate kernel (two
@@ -539,12 +515,12 @@ __global__ __launch_bounds__(128) void mla_attn_merge_kernel(int B, int H, int K
 constexpr int AO_NT = 512;                 // 8 waves, one 16-column tile of o each (VH <= 128)
 constexpr int AO_KP = 32 * 16 + 8;         // LDS row pitch (bf16): 16 bytes of skew per row
 __global__ __launch_bounds__(AO_NT) void mla_attn_out_kernel(int B, int H, int KL, int QN, int VH,
-                                                            const uint16_t *__restrict__ ch2,
+                                                            const uint16_t *__restrict__ ch3,
                                                             const uint16_t *__restrict__ kvb,
                                                             const float *__restrict__ g, long ldg,
                                                             float *__restrict__ o, float *__restrict__ zout, size_t zn)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t chh[16 * AO_KP], chl[16 * AO_KP];
+    __shared__ __attribute__((aligned(16))) uint16_t chs[3][16 * AO_KP];
     const int h = blockIdx.x, b0 = blockIdx.y * 16, nb = min(16, B - b0), tid = threadIdx.x;
     const int lane = tid & 63, wv = tid >> 6;
     const int r16 = lane & 15, kq = lane >> 4;
@@ -567,19 +543,18 @@ __global__ __launch_bounds__(AO_NT) void mla_attn_out_kernel(int B, int H, int K
 #pragma unroll
         for (int e = 0; e < 4; e++)
             if (4 * kq + e < nb) gv[e] = g[(size_t)(b0 + 4 * kq + e) * ldg + (size_t)h * VH + n];
-    // the block's chat rows (hi and lo) into LDS, 8 bf16 per thread and pass; rows past nb and
+    // the block's chat rows (all three parts) into LDS, 8 bf16 per thread and pass; rows past nb and
     // channels past KL are zero
     const size_t BN = (size_t)B * H * KL;
     for (int it = tid; it < 16 * (KLr / 8); it += AO_NT) {
         const int r = it / (KLr / 8), c = 8 * (it % (KLr / 8));
-        uint4 vh = {0, 0, 0, 0}, vl = {0, 0, 0, 0};
-        if (r < nb && c < KL) {
-            const size_t i = ((size_t)(b0 + r) * H + h) * KL + c;
-            vh = *reinterpret_cast<const uint4 *>(ch2 + i);
-            vl = *reinterpret_cast<const uint4 *>(ch2 + BN + i);
-        }
-        *reinterpret_cast<uint4 *>(chh + r * AO_KP + c) = vh;
-        *reinterpret_cast<uint4 *>(chl + r * AO_KP + c) = vl;
+        uint4 v[3];
+        const size_t i = ((size_t)(b0 + r) * H + h) * KL + c;
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+            v[p] = r < nb && c < KL ? *reinterpret_cast<const uint4 *>(ch3 + p * BN + i) : uint4{0, 0, 0, 0};
+#pragma unroll
+        for (int p = 0; p < 3; p++) *reinterpret_cast<uint4 *>(chs[p] + r * AO_KP + c) = v[p];
     }
     if (zout) {
         const size_t nwg = (size_t)gridDim.x * gridDim.y, id = (size_t)blockIdx.y * gridDim.x + h;
@@ -593,10 +568,10 @@ __global__ __launch_bounds__(AO_NT) void mla_attn_out_kernel(int B, int H, int K
     for (int ks = 0; ks < AT_MAXCT / 2; ks++) {
         if (32 * ks >= KLr) break;
         const int k = 32 * ks + 8 * kq;
-        const bf16x8 ah = *reinterpret_cast<const bf16x8 *>(chh + r16 * AO_KP + k);
-        const bf16x8 al = *reinterpret_cast<const bf16x8 *>(chl + r16 * AO_KP + k);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, wf[ks], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, wf[ks], acc, 0, 0, 0);
+#pragma unroll
+        for (int p = 2; p >= 0; p--)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8 *>(chs[p] + r16 * AO_KP + k),
+                                                          wf[ks], acc, 0, 0, 0);
     }
     // C layout: lane holds rows 4 kq + e (sequences), column r16 (value channel n)
 #pragma unroll
@@ -625,25 +600,34 @@ int at_cus()
 
 bool at_geom(int H, int KL, int CW, AtGeom &g)
 {
-    if (H <= 0 || H > 64 || KL <= 0 || (KL % 16) || KL > 16 * AT_MAXCT || CW < KL || (CW % 4) ||
+    if (H <= 0 || KL <= 0 || (KL % 16) || KL > 16 * AT_MAXCT || CW < KL || (CW % 4) ||
         CW > 32 * AT_MAXKS)
         return false;
+    const int tiles = (H + 15) / 16, groups = (tiles + 3) / 4;
+    if (groups > 65535) return false;
     g.H = H;
+    g.HG = 16 * ((tiles + groups - 1) / groups);
     g.CW = CW;
     g.KL = KL;
     return true;
 }
 
-int at_nsplit(int B, int Tn)
+// One workgroup per CU at most: a count rounded up (24 sequences: 264 workgroups) runs a
+// second, nearly empty round. With several head groups, ranges a multiple of 8, so that the
+// groups of a range run on one XCD and share its L2's copy of the cache rows.
+int at_nsplit(int B, int H, int Tn)
 {
-    return std::min({AT_MAXSPLIT, std::max(1, (at_cus() + B - 1) / B), std::max(1, Tn / AT_T)});
+    const int groups = ((H + 15) / 16 + 3) / 4;
+    int n = std::min({AT_MAXSPLIT, (int)std::max(1L, at_cus() / ((long)B * groups)), std::max(1, Tn / AT_T)});
+    if (groups > 1 && n > 8) n &= ~7;
+    return n;
 }
 
 }  // namespace
 
 size_t mla_attention_ws_bytes(int B, int H, int KL, int Tn)
 {
-    const int nsplit = at_nsplit(B, Tn);
+    const int nsplit = at_nsplit(B, H, Tn);
     const size_t r = (size_t)B * nsplit * H;
     return ((r * KL * 4 + 255) & ~(size_t)255) + 2 * ((r * 4 + 255) & ~(size_t)255);
 }
@@ -654,46 +638,41 @@ bool mla_attention_supported(int H, int KL, int CW)
     return at_geom(H, KL, CW, g);
 }
 
-int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, const float *q,
-                  int QN, float *cache, const float *lat, long ldlat, const float *lat_w, float lat_eps,
-                  const uint16_t *kvb, int VH, const float *gate, long ldg, float *o, float *zout, size_t zn,
-                  uint16_t *ch2, void *ws, size_t ws_bytes, hipStream_t st)
+int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, int planes, const float *q,
+                  int QN, const float *cache, const uint16_t *kvb, int VH, const float *gate, long ldg, float *o, float *zout, size_t zn,
+                  uint16_t *ch3, void *ws, size_t ws_bytes, hipStream_t st)
 {
     AtGeom g;
     if (!at_geom(H, KL, CW, g))
         K3_FAIL(K3HIP_EUNSUPPORTED, "mla attention: heads=%d kv_lora=%d kv_lora+rope=%d outside the fused kernel", H, KL, CW);
     if (B <= 0 || Tn <= 0 || Tn > cap) K3_FAIL(K3HIP_EINVAL, "mla attention: B=%d Tn=%d cap=%d", B, Tn, cap);
-    const int nsplit = at_nsplit(B, Tn);
+    const int nsplit = at_nsplit(B, H, Tn);
     const size_t need = mla_attention_ws_bytes(B, H, KL, Tn);
     const int QH = QN + (CW - KL);
     if (!ws || ws_bytes < need || ((uintptr_t)ws & 255) || ((uintptr_t)cache & 15) || ((uintptr_t)A2 & 15) ||
-        ((uintptr_t)q & 15) || (QN & 3) || (KL & 7) || ((uintptr_t)kvb & 15) || ((uintptr_t)ch2 & 15) ||
+        ((uintptr_t)q & 15) || (QN & 3) || (KL & 7) || ((uintptr_t)kvb & 15) || ((uintptr_t)ch3 & 15) ||
         VH < 1 || VH > 16 * (AO_NT / 64))
         K3_FAIL(K3HIP_EINVAL, "mla attention: workspace %zu < %zu bytes, or a misaligned buffer", ws_bytes, need);
-    const AtQ qs{A2, q, B, QN, QH};
-    const AtRow nr{lat, ldlat, lat_w, lat_eps, Tn - 1};
+    const AtQ qs{A2, q, planes, B, QN, QH};
     const size_t r = (size_t)B * nsplit * H;
     float *pctx = (float *)ws;
     float *pm = (float *)((char *)ws + ((r * KL * 4 + 255) & ~(size_t)255));
     float *pl = (float *)((char *)pm + ((r * 4 + 255) & ~(size_t)255));
-    static bool attr = false;
-    if (!attr) {
-        K3_HIP(hipFuncSetAttribute((const void *)mla_attn_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)AT_LDS));
-        K3_HIP(hipFuncSetAttribute((const void *)mla_attn_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)AT_LDS));
-        attr = true;
-    }
-    if (CW == 32 * AT_MAXKS)
-        hipLaunchKernelGGL(mla_attn_kernel<true>, dim3(nsplit, B), dim3(AT_NT), AT_LDS, st, g, Tn, cap, nsplit,
-                           scale * AT_LOG2E, qs, nr, cache, pctx, pm, pl);
-    else
-        hipLaunchKernelGGL(mla_attn_kernel<false>, dim3(nsplit, B), dim3(AT_NT), AT_LDS, st, g, Tn, cap, nsplit,
-                           scale * AT_LOG2E, qs, nr, cache, pctx, pm, pl);
+    const int nht = g.HG / 16, groups = (H + g.HG - 1) / g.HG;
+    const void *kern;   // more than one group: three or four head tiles each
+#define K3_AT(F) (groups > 1 ? (nht == 3 ? (const void *)mla_attn_kernel<F, 3, true> : (const void *)mla_attn_kernel<F, 4, true>) \
+                  : nht == 1 ? (const void *)mla_attn_kernel<F, 1, false> : nht == 2 ? (const void *)mla_attn_kernel<F, 2, false> \
+                  : nht == 3 ? (const void *)mla_attn_kernel<F, 3, false> : (const void *)mla_attn_kernel<F, 4, false>)
+    kern = CW == 32 * AT_MAXKS ? K3_AT(true) : K3_AT(false);
+#undef K3_AT
+    K3_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)AT_LDS));
+    float scale2 = scale * AT_LOG2E;
+    void *args[] = {&g, &Tn, &cap, (void *)&nsplit, &scale2, (void *)&qs, (void *)&cache, &pctx, &pm, &pl};
+    K3_HIP(hipLaunchKernel(kern, dim3(nsplit, B, groups), dim3(AT_NT), args, AT_LDS, st));
     K3_LAUNCHED();
-    hipLaunchKernelGGL(mla_attn_merge_kernel, dim3(H, B), dim3(128), 0, st, B, H, KL, nsplit, pctx, pm, pl, ch2);
+    hipLaunchKernelGGL(mla_attn_merge_kernel, dim3(H, B), dim3(128), 0, st, B, H, KL, nsplit, pctx, pm, pl, ch3);
     K3_LAUNCHED();
-    hipLaunchKernelGGL(mla_attn_out_kernel, dim3(H, (B + 15) / 16), dim3(AO_NT), 0, st, B, H, KL, QN, VH, ch2, kvb,
+    hipLaunchKernelGGL(mla_attn_out_kernel, dim3(H, (B + 15) / 16), dim3(AO_NT), 0, st, B, H, KL, QN, VH, ch3, kvb,
                        gate, ldg, o, zout, zn);
     K3_LAUNCHED();
     return K3HIP_OK;

@@ -16,9 +16,11 @@
 // batch-16 KDA decode layer at hidden 7168 measured 97.5 -> 83.2 us with them.
 //
 // Precision: x stays fp32. Each 8-element slice of an x row is split in registers into
-// bf16 hi + lo (x = hi + lo to ~2^-17 relative), and both halves go through the same bf16
-// MFMA against the bf16 weight (an exact product) into one fp32 accumulator, so every
-// product keeps fp32 accuracy with no extra weight traffic.
+// bf16 hi + mid + lo (all 24 bits of x), and the three go through the same bf16 MFMA against
+// the bf16 weight (an exact product) into one fp32 accumulator, so every product keeps fp32
+// accuracy with no extra weight traffic. hi + mid alone left 2.5e-6 relative (rms) per
+// product; the third part is free while the weight's bytes bound the launch (14,400 x 7168,
+// B = 16: 34.2 us with either, B = 64: 66.3 against 64.7).
 //
 // Work split: a workgroup of 8 waves owns 64 output columns (4 column groups) and one
 // K-range; its waves take the K-steps of the range round robin. The number of K-ranges per
@@ -69,8 +71,8 @@ struct RowsJob {
     const uint16_t *Wf;
     float *P;
     long ldp, split_stride;
-    // unsplit products only: C also as bf16 hi (row m) and lo (plane hlplane on) rows of
-    // stride ldhl, x = hi + lo, for a following GEMM on split rows (nullptr: none)
+    // unsplit products only: C also as bf16 hi (row m), mid and lo (each a plane hlplane on)
+    // rows of stride ldhl, x = hi + mid + lo, for a following product on split rows (nullptr: none)
     uint16_t *hl = nullptr;
     long ldhl = 0, hlplane = 0;
 };
@@ -84,13 +86,13 @@ struct RowsJob {
 // inv = 1 / sqrt(mean_k x^2 + xeps) (mean in double; src/core/k3_ops.c:94-102), so a
 // normalised input needs no launch of its own.
 template <int MT, bool ATOM, bool NORM>
-__global__ __launch_bounds__(64 * RT_WAVES) void rows_gemm_kernel(int B, int K, const float *__restrict__ x,
+__global__ __launch_bounds__(64 * RT_WAVES, MT == 4 ? 2 : 4) void rows_gemm_kernel(int B, int K, const float *__restrict__ x,
                                                                   long ldx, RowsJob j0, RowsJob j1,
                                                                   const float *__restrict__ xw, float xeps)
 {
     __shared__ f32x4 red[RT_WAVES][RT_NT][MT][64];
     __shared__ float xinv[16 * MT];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, kg = lane >> 4;
     const int n0 = j0.nb * j0.S;
     const bool second = (int)blockIdx.x >= n0;
@@ -118,14 +120,32 @@ __global__ __launch_bounds__(64 * RT_WAVES) void rows_gemm_kernel(int B, int K, 
         xrow[mt] = x + (size_t)min(16 * mt + r16, B - 1) * ldx;
     }
 
-    // with a normalised input, this wave's first weight fragments are requested before the
-    // rows' inverse RMS is formed, so that their latency hides behind it
-    bf16x8 wv0[RT_NT];
-    const int t0 = tbeg + w;
-    if (NORM && t0 < tend) {
+    // One K-step's weight fragments and x slices, all requested before any is used: left to
+    // itself the scheduler sinks some of the weight loads behind the wait for x, two memory
+    // latencies per K-step (14,400 x 7168, 225 workgroups, B = 16: 44.7 us against 34.2, a
+    // plain read of the weight 33.6). Keeping the next step's loads in flight as well gave
+    // 35.0, and 76 against 43 at B = 32 (registers).
+    struct Step {
+        bf16x8 wv[RT_NT];
+        f4 xa[MT], xb[MT];
+    };
+    auto load_step = [&](Step &st, int t) {
+        const int k = 32 * t + 8 * kg;   // K % 8 == 0: the 8-slice is wholly inside or outside
+        const int kk = k < K ? k : 0;
 #pragma unroll
-        for (int j = 0; j < RT_NT; j++) wv0[j] = __builtin_nontemporal_load(&wg[j][(size_t)t0 * 64]);
-    }
+        for (int mt = 0; mt < MT; mt++) {
+            st.xa[mt] = *reinterpret_cast<const f4 *>(xrow[mt] + kk);
+            st.xb[mt] = *reinterpret_cast<const f4 *>(xrow[mt] + kk + 4);
+        }
+#pragma unroll
+        for (int j = 0; j < RT_NT; j++) st.wv[j] = __builtin_nontemporal_load(&wg[j][(size_t)t * 64]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // with a normalised input, the first step is requested before the rows' inverse RMS is
+    // formed, so that its latency hides behind it
+    const int t0 = tbeg + w;
+    Step first;
+    if (NORM && t0 < tend) load_step(first, t0);
     if constexpr (NORM) {   // the rows' inverse RMS: 32 lanes per row, 16 rows per pass
         for (int rr0 = 0; rr0 < 16 * MT; rr0 += 16) {
             const int rr = rr0 + ((int)threadIdx.x >> 5), ln = threadIdx.x & 31;
@@ -159,42 +179,39 @@ __global__ __launch_bounds__(64 * RT_WAVES) void rows_gemm_kernel(int B, int K, 
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) acc[j][mt] = 0.0f;
 
-    for (int t = t0; t < tend; t += RT_WAVES) {
-        bf16x8 wv[RT_NT];
-        if (NORM && t == t0) {
-#pragma unroll
-            for (int j = 0; j < RT_NT; j++) wv[j] = wv0[j];
-        } else {
-#pragma unroll
-            for (int j = 0; j < RT_NT; j++) wv[j] = __builtin_nontemporal_load(&wg[j][(size_t)t * 64]);
-        }
-        const int k = 32 * t + 8 * kg;   // K % 8 == 0: the 8-slice is wholly inside or outside
+    auto step = [&](const Step &st, int t) {
+        const int k = 32 * t + 8 * kg;
         const bool kin = k < K;
-        f4 xa[MT], xb[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            xa[mt] = *reinterpret_cast<const f4 *>(xrow[mt] + (kin ? k : 0));
-            xb[mt] = *reinterpret_cast<const f4 *>(xrow[mt] + (kin ? k : 0) + 4);
-        }
+        f4 wa = 0.0f, wb = 0.0f;
         if constexpr (NORM) {
-            const f4 wa = *reinterpret_cast<const f4 *>(xw + (kin ? k : 0));
-            const f4 wb = *reinterpret_cast<const f4 *>(xw + (kin ? k : 0) + 4);
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                xa[mt] = (wa * xa[mt]) * xiv[mt];
-                xb[mt] = (wb * xb[mt]) * xiv[mt];
-            }
+            wa = *reinterpret_cast<const f4 *>(xw + (kin ? k : 0));
+            wb = *reinterpret_cast<const f4 *>(xw + (kin ? k : 0) + 4);
         }
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-            bf16x8 xh, xl;
-            const bool ok = kin && xlive[mt];
-            split_row8(ok ? xa[mt] : f4(0.0f), ok ? xb[mt] : f4(0.0f), xh, xl);
-#pragma unroll
-            for (int j = 0; j < RT_NT; j++) {
-                acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, wv[j], acc[j][mt], 0, 0, 0);
-                acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, wv[j], acc[j][mt], 0, 0, 0);
+            f4 xa = st.xa[mt], xb = st.xb[mt];
+            if constexpr (NORM) {
+                xa = (wa * xa) * xiv[mt];
+                xb = (wb * xb) * xiv[mt];
             }
+            bf16x8 xh, xm, xl;
+            const bool ok = kin && xlive[mt];
+            split_row8(ok ? xa : f4(0.0f), ok ? xb : f4(0.0f), xh, xm, xl);
+#pragma unroll
+            for (int j = 0; j < RT_NT; j++) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, st.wv[j], acc[j][mt], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < RT_NT; j++) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xm, st.wv[j], acc[j][mt], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < RT_NT; j++) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, st.wv[j], acc[j][mt], 0, 0, 0);
+        }
+    };
+    for (int t = t0; t < tend; t += RT_WAVES) {
+        if (NORM && t == t0) {
+            step(first, t);
+        } else {
+            Step st;
+            load_step(st, t);
+            step(st, t);
         }
     }
 
@@ -221,9 +238,10 @@ __global__ __launch_bounds__(64 * RT_WAVES) void rows_gemm_kernel(int B, int K, 
                 } else {
                     out[(size_t)m * ldp + n] = t[e];
                     if (jb.hl) {
-                        const uint16_t hi = f2bf(t[e]);
-                        jb.hl[(size_t)m * jb.ldhl + n] = hi;
-                        jb.hl[(size_t)jb.hlplane + (size_t)m * jb.ldhl + n] = f2bf(t[e] - __uint_as_float((uint32_t)hi << 16));
+                        uint16_t h3[3];
+                        split3(t[e], h3);
+#pragma unroll
+                        for (int p = 0; p < 3; p++) jb.hl[(size_t)p * jb.hlplane + (size_t)m * jb.ldhl + n] = h3[p];
                     }
                 }
             }
@@ -428,7 +446,7 @@ int gemm_rows_hl(int B, int N, int K, const float *x, long ldx, const uint16_t *
         int rc = gemm_rows(B, N, K, x, ldx, Wf, C, ldc, st, ws, ws_floats);
         if (rc) return rc;
         if (ldhl != N || ldc != N) K3_FAIL(K3HIP_EINVAL, "gemm_rows_hl: a split-K product needs ldc = ldhl = N");
-        return split_rows2(C, hl, B, N, st);
+        return split_rows3(C, hl, B, N, st);
     }
     if ((K & 7) || (ldx & 3) || (((uintptr_t)x | (uintptr_t)Wf) & 15))
         K3_FAIL(K3HIP_EINVAL, "gemm_rows_hl: K=%d ldx=%ld need multiples of 8 / 4 and 16-byte aligned x, W", K, ldx);

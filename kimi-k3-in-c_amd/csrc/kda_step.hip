@@ -35,7 +35,7 @@
 //
 // In the layer form, the decay logits z = f_a . W_fb^T (the f_b projection, k3_ops.c:886, D
 // outputs of the head from the D-wide f_a row) are computed here too, one 16-channel group of W_fb per
-// wave, in the arithmetic of the decode GEMV (kda_rows.hip): f_a split into bf16 hi + lo
+// wave, in the arithmetic of the decode GEMV (kda_rows.hip): f_a split into bf16 hi + mid + lo
 // against the bf16 weight fragments, each 32-wide K-step's product an fp32 partial of its
 // own, the partials added in K-step order. z gets the bits the stand-alone GEMV gives it,
 // without its launch and its round trip through memory (batch-16 decode layer at hidden
@@ -206,9 +206,10 @@ __global__ __launch_bounds__(4 * D) void kda_layer_step_kernel(const StepArgs a)
         f32x4 zs = 0.0f;
 #pragma unroll
         for (int t = 0; t < KT; t++) {
-            bsplit::bf16x8 xh, xl;
-            bsplit::split_row8(fxa[t], fxb[t], xh, xl);
+            bsplit::bf16x8 xh, xm, xl;
+            bsplit::split_row8(fxa[t], fxb[t], xh, xm, xl);
             f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, wfr[t], f32x4(0.0f), 0, 0, 0);
+            p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xm, wfr[t], p, 0, 0, 0);
             p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, wfr[t], p, 0, 0, 0);
             zs = t == 0 ? p : zs + p;
         }
