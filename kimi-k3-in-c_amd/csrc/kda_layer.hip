@@ -469,6 +469,15 @@ extern "C" int k3hip_kda_upload_ex(const K3KdaW *w, const K3Cfg *c, int parts, k
 // recurrence.
 static bool chunk_gate_ok(float lb) { return lb < 0.0f && fabsf(lb) * 15.0f <= 80.0f; }
 
+// Where k3hip_kda_layer_dev runs its bf16 projections. Fewer than 33 tokens: the double products
+// of kda_proj.hip, no slower there and more accurate (hidden 1024, 8 x 64 heads T = 24: 40 us
+// against 50; hidden 4096, 32 x 128: 163 | 153, but T = 36 already 213 | 155). Then
+// kda_mid.hip up to MID_DEV_MACS products of the input projections (hidden 4096, 32 x 128 heads
+// T = 333: 775 -> 249 us, T = 3000 (2.0e11) 1622 -> 1497 us; T = 8192 (5.6e11) 3933 | 4104), then
+// the 256 x 256 tiles of kda_mm.hip on 2T split rows.
+constexpr int MID_DEV_T = 33;
+constexpr double MID_DEV_MACS = 4e11;
+
 extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out, const float *x,
                                    float *state, void *stream)
 {
@@ -512,44 +521,54 @@ extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out
         if (!step) cs = nullptr;
     }
 
-    // Projections. bf16 weights on a T >= 16 prefill: MFMA GEMMs (kda_mm.hip) of the input
-    // split into bf16 hi + lo rows, the two halves' fp32 products added, so the products keep
-    // fp32 accuracy (x = hi + lo to 2^-17, bf16 x bf16 exact in fp32, fp32 sums over K) and
-    // the layer stays within the reference's 1e-4 bar. Otherwise (fp32 or int8 weights,
-    // short T, widths that are not multiples of 64) the double-accumulating GEMV.
-    const bool mfma = w->wdt == K3_WBF16 && T >= 16 && E % 64 == 0 && D % 64 == 0 && P % 64 == 0 &&
+    // Projections. bf16 weights on a T >= MID_DEV_T prefill: MFMA products of the input split into
+    // bf16 hi + lo, so the products keep fp32 accuracy (x = hi + lo to 2^-17, bf16 x bf16 exact in
+    // fp32, fp32 sums over K) and the layer stays within the reference's 1e-4 bar: split as it is
+    // read (kda_mid.hip), or the longest prefills as 2T split rows whose two halves are added.
+    // Otherwise (fp32 or int8 weights, short T, widths that are not multiples of 64) the
+    // double-accumulating products of kda_proj.hip.
+    const bool mfma = w->wdt == K3_WBF16 && T >= MID_DEV_T && E % 64 == 0 && D % 64 == 0 && P % 64 == 0 &&
                       ((uintptr_t)x & 15) == 0;
+    const bool big = mfma && (double)T * (4.0 * P + D + H) * E > MID_DEV_MACS;
     StreamBuf sbuf;
     uint16_t *xs = nullptr;
     float *C2 = nullptr;
-    if (mfma) {
-        const size_t maxin = std::max<size_t>(E, P), maxout = std::max<size_t>(E, P);
-        const size_t xsb = ((2 * (size_t)T * maxin * 2) + 255) & ~(size_t)255;
-        if ((rc = stream_alloc(sbuf, xsb + 2 * (size_t)T * maxout * 4, st))) return rc;
+    if (big) {
+        const size_t widest = std::max<size_t>(E, P);
+        const size_t xsb = ((2 * (size_t)T * widest * 2) + 255) & ~(size_t)255;
+        if ((rc = stream_alloc(sbuf, xsb + 2 * (size_t)T * widest * 4, st))) return rc;
         xs = (uint16_t *)sbuf.p;
         C2 = (float *)((char *)sbuf.p + xsb);
     }
-    // y[T][out] = in[T][nin] . W[out][nin]^T, from the split input xs when mfma
+    // y[T][out] = in[T][nin] . W[out][nin]^T, from the split input xs when big
     auto project = [&](int nin, int nout, const float *in, const void *W, float *y) -> int {
         if (!mfma) return proj(T, nin, nout, in, W, w->wdt, y, st);
+        if (!big) {
+            const MidSeg s{W, y, nout, nout};
+            return mid(T, nin, MID_A_SPLIT, in, nin, &s, 1, false, K3HIP_F32, st);
+        }
         int r = mm(2 * T, nout, nin, K3HIP_BF16, xs, nin, W, nin, C2, K3HIP_F32, nout, st);
         return r ? r : pair_add(C2, y, T, nout, st);
     };
-    if (mfma) {
+    const int iP = (int)P;
+    if (big) {
         if ((rc = split_rows2(x, xs, T, E, st))) return rc;
-        if ((rc = project(E, (int)P, x, w->q, qp))) return rc;
-        if ((rc = project(E, (int)P, x, w->k, kp))) return rc;
-        if ((rc = project(E, (int)P, x, w->v, vp))) return rc;
+        if ((rc = project(E, iP, x, w->q, qp))) return rc;
+        if ((rc = project(E, iP, x, w->k, kp))) return rc;
+        if ((rc = project(E, iP, x, w->v, vp))) return rc;
         if ((rc = project(E, H, x, w->b, bl))) return rc;
         if ((rc = project(E, D, x, w->f_a, fa))) return rc;
-        if ((rc = project(E, (int)P, x, w->g, gl))) return rc;
+        if ((rc = project(E, iP, x, w->g, gl))) return rc;
         if ((rc = split_rows2(fa, xs, T, D, st))) return rc;
+    } else if (mfma) {
+        const MidSeg in[5] = {{w->q, qp, iP, iP}, {w->k, kp, iP, iP}, {w->v, vp, iP, iP}, {w->g, gl, iP, iP},
+                              {w->f_a, fa, D, D + H, D, bl, H}};
+        if ((rc = mid(T, E, MID_A_SPLIT, x, E, in, 5, false, K3HIP_F32, st))) return rc;
     } else {
-        const ProjSeg in[6] = {{w->q, qp, (int)P}, {w->k, kp, (int)P}, {w->v, vp, (int)P},
-                               {w->g, gl, (int)P}, {w->f_a, fa, D},    {w->b, bl, H}};
+        const ProjSeg in[6] = {{w->q, qp, iP}, {w->k, kp, iP}, {w->v, vp, iP}, {w->g, gl, iP}, {w->f_a, fa, D}, {w->b, bl, H}};
         if ((rc = proj_multi(T, E, in, 6, x, w->wdt, st))) return rc;
     }
-    if ((rc = project(D, (int)P, fa, w->f_b, z))) return rc;
+    if ((rc = project(D, iP, fa, w->f_b, z))) return rc;
 
     const float qscale = 1.0f / sqrtf((float)D);
     if (step) {
@@ -571,8 +590,8 @@ extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out
     if (rc) return rc;
     if (!step && (rc = k3hip_kda_epilogue(T, H, D, w->rms_eps, o, gl, K3HIP_F32, w->o_norm, y, K3HIP_F32, stream)))
         return rc;
-    if (mfma && (rc = split_rows2(y, xs, T, (int)P, st))) return rc;
-    return project((int)P, E, y, w->o, out);
+    if (big && (rc = split_rows2(y, xs, T, iP, st))) return rc;
+    return project(iP, E, y, w->o, out);
 }
 
 // fp32 -> bf16 (round to nearest even), for fp32 layer inputs of the bf16 prefill path.
@@ -703,6 +722,12 @@ extern "C" int k3hip_set_projection_gemm(int impl)
     return K3HIP_OK;
 }
 
+// Products of the input projections (T x their rows x hidden) up to which the short form of the
+// prefill runs: against the library's launches, hidden 4096 and 32 x 128 heads T = 330 (22e9)
+// 185 -> 149 us, T = 420 (28e9) 200 | 207; hidden 4096 and 16 x 64 heads T = 1400 (24e9) 207 ->
+// 152; hidden 2048 and 48 x 128 heads T = 450 (23e9) 222 -> 192, T = 700 (36e9) 272 | 280.
+constexpr double MID_PREFILL_MACS = 24e9;
+
 extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *out, int out_dtype,
                                        const void *x, int x_dtype, float *state, void *stream)
 {
@@ -738,15 +763,17 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
                      mm_supported(E, E, E) && (x_dtype == K3HIP_F32 || ((uintptr_t)x & 15) == 0);
     int ncu = 256, rc;
     if ((rc = cu_count(ncu))) return rc;
+    // Short prefills: all input projections in one launch, z and o_proj in one each (kda_mid.hip).
+    const bool sh = !own && (double)T * (4.0 * P + D + H) * E <= MID_PREFILL_MACS && mid_supported(E, x_dtype == K3HIP_F32 ? nullptr : x, E, false);
     const int fab_s = own ? mm_splits(T, D + H, E, ncu) : 1;
     // scratch, 256-byte aligned pieces:
     //   0 x bf16 | 1 q k v projections fp32 | 2 f_a and b fp32 (split-K planes) | 3 f_a hi/lo bf16 |
     //   4 z fp32 | 5 b logits | 6 o fp32 | 7 gate fp16 | 8 y fp16 | 9 zero state | 10 chunk workspace |
-    //   11 fp32 o_proj result (fallback path with a bf16 out)
+    //   11 fp32 o_proj result (library path with a bf16 out) | 12 gate fp32 (short prefills)
     size_t sizes[] = {x_dtype == K3HIP_F32 ? (size_t)T * E * 2 : 0, 3 * TP * 4, (size_t)fab_s * T * (D + H) * 4,
                       (size_t)T * D * 4, TP * 4, (size_t)T * H * 4, TP * 4, TP * 2, TP * 2,
                       state ? 0 : (size_t)H * D * D * 4, wsb,
-                      (!own && out_dtype == K3HIP_BF16) ? (size_t)T * E * 4 : 0};
+                      (!own && !sh && out_dtype == K3HIP_BF16) ? (size_t)T * E * 4 : 0, sh ? TP * 4 : 0};
     constexpr int NB = sizeof sizes / sizeof sizes[0];
     size_t off[NB], total = 0;
     for (int i = 0; i < NB; i++) {
@@ -784,7 +811,16 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
     //   2e-3 bar): q, k, v as one GEMM over their consecutive weight rows, its three column
     //   groups written to three [T][P] arrays; f_a and b as one split-K GEMM whose reduction
     //   writes f_a as a bf16 hi/lo pair for z = [f_a_hi | f_a_lo] [W_fb | W_fb]^T (fp32 accuracy)
-    if (own) {
+    const int iP = (int)P;
+    float *gl = sh ? (float *)(base + off[12]) : z;   // the library path's gate takes z's place, consumed by then
+    if (sh) {
+        // f_a stays fp32; the z product splits it as it reads it
+        const MidSeg in[5] = {{w->q, qp, iP, iP}, {w->k, kp, iP, iP}, {w->v, vp, iP, iP}, {w->g, gl, iP, iP},
+                              {w->f_a, fa, D, D + H, D, bl, H}};
+        const MidSeg zs{w->f_b, z, iP, iP};
+        if ((rc = mid(T, E, MID_A_16, xb, E, in, 5, false, K3HIP_F32, st))) return rc;
+        if ((rc = mid(T, D, MID_A_SPLIT, fa, D, &zs, 1, false, K3HIP_F32, st))) return rc;
+    } else if (own) {
         if ((rc = mm(T, 3 * (int)P, E, K3HIP_BF16, xb, E, wq, E, qp, K3HIP_F32, (long)P, st, (int)P, (long)TP)))
             return rc;
         if ((rc = mm_splitk(T, D + H, E, fab_s, K3HIP_BF16, xb, E, w->f_a, E, fa, st))) return rc;
@@ -822,11 +858,14 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
         // 9 o_proj on fp16 MFMA against the fp16 copy of W_o
         return mm(T, E, (int)P, K3_DT_F16, y16, (long)P, w->o16, (long)P, out, out_dtype, E, st);
     }
-    // hipBLASLt has no bf16-in, fp16-out algorithm: this path keeps fp32 gate logits (z is
-    // consumed by now)
-    float *gl = z;
-    if ((rc = gemm_bf16(T, (int)P, E, xb, w->g, gl, K3HIP_F32, st))) return rc;
+    // hipBLASLt has no bf16-in, fp16-out algorithm: this path keeps fp32 gate logits, as the
+    // short one does
+    if (!sh && (rc = gemm_bf16(T, iP, E, xb, w->g, gl, K3HIP_F32, st))) return rc;
     if ((rc = epilogue_split(T, H, D, w->rms_eps, o, gl, K3HIP_F32, w->o_norm, y16, st, true))) return rc;
+    if (sh) {
+        const MidSeg os{w->o16, out, E, E};
+        return mid(T, iP, MID_A_16, y16, iP, &os, 1, true, out_dtype, st);
+    }
     if (out_dtype == K3HIP_F32) return gemm_f16(T, E, (int)P, y16, w->o16, out, K3HIP_F32, st);
     float *o32 = (float *)(base + off[11]);
     if ((rc = gemm_f16(T, E, (int)P, y16, w->o16, o32, K3HIP_F32, st))) return rc;

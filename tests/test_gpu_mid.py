@@ -1,0 +1,67 @@
+# SPDX-License-Identifier: Apache-2.0
+"""The short-prefill projections (csrc/kda_mid.hip) where they can go wrong: one K-step, row
+counts around the 64- and 128-row tiles, head counts whose q / k / v / gate blocks end inside a
+column tile, each tile shape (64 x 64; 64 x 128; 128 x 128 from 256 tiles on), bf16 and fp32
+inputs and results. Held, like the other forms, to the oracle's k3_kda_layer: the bf16 prefill at
+2e-3 (its bf16 results at twice that, the rounding of the result), the full-accuracy layer on
+bf16 weights at 1e-4, the projected inputs in the conv history at 1e-5 (fp32 sums).
+
+The full-accuracy layer's S is held in the 2-norm, at 3e-5: the split products (hi + lo of each
+operand, 2.5e-6 rms each, lo x lo left out, in the projections, the chunk factors and the state
+update) put it 6e-6 to 8e-6 from 64 bits at these shapes, in any order of the sums. Element by
+element against the rms of all heads that spread has no fixed bound: the rows of a head's slowly
+decaying channels are many times the rms, and so are their errors (half a million elements at
+32 x 128 heads)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import assert_close
+from test_gpu_layer_prefill import TOL, bf16_to_f32, layer_weights, rms
+from test_oracle_ref import bf16
+import k3_oracle as ko
+from k3_oracle import f32
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(64, 3, 64, (33, 64, 65)), (192, 5, 64, (127, 129)), (128, 2, 128, (40, 200)),
+          (64, 32, 128, (63, 257)), (1024, 33, 64, (97,))]
+
+
+@pytest.mark.parametrize("dev", [False, True])
+@pytest.mark.parametrize("hidden,H,D,Ts", SHAPES)
+def test_short_prefill_projections_vs_oracle(gpu, hidden, H, D, Ts, dev):
+    import torch
+    rng = np.random.default_rng(0x4B334441 + 0x1D + hidden + H)
+    K, P = 4, H * D
+    W = layer_weights(rng, hidden, H, D, K)
+    cfg = ko.make_cfg(hidden, H, D, K, -5.0, 1e-5)
+    nst = P * D + 3 * P * (K - 1)
+    st_ref = np.zeros(nst, np.float32)
+    dw = gpu.DeviceWeights(W.w, cfg, gpu.UPLOAD_DEV if dev else gpu.UPLOAD_PREFILL)
+    dst = torch.zeros(nst, device="cuda")
+    for i, T in enumerate(Ts):
+        x = f32(rng.standard_normal((T, hidden)))
+        if not dev:
+            x = bf16_to_f32(bf16(x))
+        want = ko.kda_layer(ko.orc(), x, W, cfg, T, st_ref)
+        dx = torch.from_numpy(x).cuda()
+        half = not dev and i % 2 == 1                       # bf16 results
+        out = torch.full((T, hidden), float("nan"), device="cuda", dtype=torch.bfloat16 if half else torch.float32)
+        if dev:
+            dw.layer(out, dx, dst, T)
+        else:
+            dw.layer_prefill(out, dx.to(torch.bfloat16) if (i + H) % 2 else dx, dst, T)
+        torch.cuda.synchronize()
+        tol = 1e-4 if dev else (2 * TOL if half else TOL)
+        r = assert_close(out.float().cpu().numpy(), want, tol * rms(want), tol, f"T={T} out")
+        got = dst.cpu().numpy()
+        if dev:
+            e = np.linalg.norm(np.float64(got[:P * D]) - st_ref[:P * D]) / np.linalg.norm(np.float64(st_ref[:P * D]))
+            assert e <= 3e-5, f"T={T} S: {e:.2e} from the oracle"
+        else:
+            assert_close(got[:P * D], st_ref[:P * D], TOL * rms(st_ref[:P * D]), TOL, f"T={T} S")
+        assert_close(got[P * D:], st_ref[P * D:], 1e-5 * rms(st_ref[P * D:]), 1e-5, f"T={T} conv history")
+        print(f"hidden={hidden} H={H} D={D} T={T} {'dev' if dev else 'prefill'}: worst {r:.3f}x", flush=True)
+    dw.close()
