@@ -130,12 +130,15 @@ __device__ __forceinline__ void store_cpl(float *p, const float (&v)[CPL])
     else *reinterpret_cast<f2 *>(p) = f2{v[0], v[1]};
 }
 
-// Workspace stores: 16-byte buffer stores with the system-scope non-temporal policy
-// (aux 19 = sc0 | nt | sc1: through to memory, kept in no cache), addressed from the item's
-// block. The workspace is read back by the next kernel from HBM (its L2 warm-up touches) and
-// is larger than the memory-side cache, so keeping any of it only displaces the inputs: phase
-// 1 at T=8192, H=32, D=128 -5 us with the compiler's nontemporal stores, and the core step
-// 0.5355 -> 0.5333 ms with this policy. They are compiler-visible stores, so the wait states
+// Workspace stores: 16-byte buffer stores addressed from the item's block. A pass whose
+// workspace does not fit the 256 MB memory-side cache (KEEP false) stores with the system-scope
+// non-temporal policy (aux 19 = sc0 | nt | sc1: through to memory, kept in no cache): the next
+// kernel reads it back from HBM (its L2 warm-up touches), and keeping any of it only displaces
+// the inputs (phase 1 at T=8192, H=32, D=128 -5 us with the compiler's nontemporal stores, and
+// the core step 0.5355 -> 0.5333 ms with this policy; ordinary stores 0.533 against 0.521). A
+// smaller one (KEEP) is stored ordinarily and found in that cache: T=701, 6 x 64 heads 35.1 ->
+// 32.0 us; T=2048, 32 x 128 (151 MB) 144.3 -> 140.6; T=5000, 8 x 128 188 -> 167; the two meet
+// at 250 MB (T=3400, 32 x 128: 233.3 | 233.8). They are compiler-visible stores, so the wait states
 // a store needs (an MFMA result as data, a VALU overwrite of its data registers) are inserted
 // as for any other.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t ws_rsrc(char *blk, size_t bytes)
@@ -143,21 +146,24 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t ws_rsrc(char *blk, size_t byte
     return __builtin_amdgcn_make_buffer_rsrc(blk, (short)0, (int)bytes, 0x00020000);
 }
 
-template <typename V>
+constexpr size_t WS_CACHED_BYTES = 200u << 20;
+
+template <bool KEEP, typename V>
 __device__ __forceinline__ void store_ws(__amdgpu_buffer_rsrc_t r, int off, const V &v)
 {
     static_assert(sizeof(V) == 16, "16-byte stores");
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, 19);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, KEEP ? 0 : 19);
 }
 
 // Split x and store it as lane `lane` of the fragment block `off` bytes into the item's block.
+template <bool KEEP>
 __device__ __forceinline__ void store_frag(__amdgpu_buffer_rsrc_t r, int off, int lane, const float (&x)[8])
 {
     bf16x8 hi, lo;
     split8(x, hi, lo);
-    store_ws(r, off + lane * 16, hi);
-    store_ws(r, off + 1024 + lane * 16, lo);
+    store_ws<KEEP>(r, off + lane * 16, hi);
+    store_ws<KEEP>(r, off + 1024 + lane * 16, lo);
 }
 
 struct Frag {
@@ -218,7 +224,7 @@ __device__ __forceinline__ void zero_upper(float *sT, int tid)
 // hook(0) .. hook(6) are called between the stages; the fused kernel issues its prefetch of
 // the next item's inputs in parts there, so that the loads of all workgroups spread over the
 // item instead of reaching HBM as one burst.
-template <int D, typename Hook>
+template <int D, bool KEEP, typename Hook>
 __device__ __forceinline__ void p1_item(float *lds, const float (&vreg)[2][8], char *blk, Hook &&hook)
 {
     using L = P1Lds<D>;
@@ -281,7 +287,7 @@ __device__ __forceinline__ void p1_item(float *lds, const float (&vreg)[2][8], c
                 const int s = 32 * ks + 8 * kg + e;
                 x[e] = sK[s * PD + i] * exp2_fast(gl - sG[s * PD + i]);
             }
-            store_frag(wr, (int)WL::KF + fb * 2048, lane, x);
+            store_frag<KEEP>(wr, (int)WL::KF + fb * 2048, lane, x);
         }
     } else {
         // wave -> (row block a, first column block b0, column blocks nb)
@@ -343,7 +349,7 @@ __device__ __forceinline__ void p1_item(float *lds, const float (&vreg)[2][8], c
         const int fb = tid >> 6, rt = fb >> 1, ks = fb & 1;
         float x[8];
         lds8(x, &sT[(SB * rt + m) * PA + 32 * ks + 8 * kg]);
-        store_frag(wr, (int)WL::AF + fb * 2048, lane, x);
+        store_frag<KEEP>(wr, (int)WL::AF + fb * 2048, lane, x);
     }
     __syncthreads();   // the inverse below overwrites every block of sT at or below the diagonal
 
@@ -419,7 +425,7 @@ __device__ __forceinline__ void p1_item(float *lds, const float (&vreg)[2][8], c
             lds8(gx, &sG[t * PD + i0]);
 #pragma unroll
             for (int e = 0; e < 8; e++) x[e] = x[e] * exp2_fast(gx[e]);
-            store_frag(wr, (int)WL::QF + fb * 2048, lane, x);
+            store_frag<KEEP>(wr, (int)WL::QF + fb * 2048, lane, x);
         }
     }
     __syncthreads();
@@ -493,7 +499,7 @@ __device__ __forceinline__ void p1_item(float *lds, const float (&vreg)[2][8], c
         }
 #pragma unroll
         for (int a = 0; a < 4; a++) {
-            store_ws(wr, (int)WL::UC + ((a * NCT + nt) * 64 + lane) * 16, au[a]);
+            store_ws<KEEP>(wr, (int)WL::UC + ((a * NCT + nt) * 64 + lane) * 16, au[a]);
 #pragma unroll
             for (int e = 0; e < 4; e++) sX[(SB * a + 4 * kg + e) * PD + n0 + m] = aw[a][e];
         }
@@ -506,7 +512,7 @@ __device__ __forceinline__ void p1_item(float *lds, const float (&vreg)[2][8], c
         const int fb = f >> 6, rt = fb / KSI, ks = fb % KSI;
         float x[8];
         lds8(x, &sX[(SB * rt + m) * PD + 32 * ks + 8 * kg]);
-        store_frag(wr, (int)WL::WF + fb * 2048, lane, x);
+        store_frag<KEEP>(wr, (int)WL::WF + fb * 2048, lane, x);
     }
 
     hook(6);
@@ -520,7 +526,7 @@ __device__ __forceinline__ void p1_item(float *lds, const float (&vreg)[2][8], c
 // into registers while the current item computes; their row indices are clamped into the
 // sequence and padding rows are zeroed only when the values are consumed, so no
 // instruction waits on these loads before the next item.
-template <int D>
+template <int D, bool KEEP>
 __global__ __launch_bounds__(P1_THREADS) void kda_chunk_intra(int T, int H, float qs,
                                                               const float *__restrict__ q,
                                                               const float *__restrict__ k,
@@ -590,7 +596,7 @@ __global__ __launch_bounds__(P1_THREADS) void kda_chunk_intra(int T, int H, floa
         if (tid < CH) sB[tid] = tid < Tc ? pb : 0.0f;
         __syncthreads();
         fetch(min(item + (int)gridDim.x, nitems - 1));
-        p1_item<D>(lds, vreg, blk_addr<D>(ws, c, H, h), [](int) {});
+        p1_item<D, KEEP>(lds, vreg, blk_addr<D>(ws, c, H, h), [](int) {});
     }
 }
 
@@ -610,7 +616,7 @@ __global__ __launch_bounds__(P1_THREADS) void kda_chunk_intra(int T, int H, floa
 // Persistent over a contiguous range of items in head-major order (item = head * nch +
 // chunk), so a workgroup keeps one head -- its conv taps and dt_bias sit in LDS -- for many
 // consecutive chunks. The next item's raw rows are prefetched into registers.
-template <int D, int K, int DT>
+template <int D, int K, int DT, bool KEEP>
 __global__ __launch_bounds__(P1_THREADS) void kda_chunk_intra_act(
     int T, int H, float qs, float lb, const void *__restrict__ q_in,
     const void *__restrict__ k_in, const void *__restrict__ v_in,
@@ -787,7 +793,7 @@ __global__ __launch_bounds__(P1_THREADS) void kda_chunk_intra_act(
         __syncthreads();   // v staging read before the A/Tm area is written
         zero_upper<D>(sA + CH * L::PA, tid);
         const int next = min(item + 1, hi - 1);
-        p1_item<D>(lds, vreg, blk_addr<D>(ws, c, H, h), [&](int part) { fetch(next, part); });
+        p1_item<D, KEEP>(lds, vreg, blk_addr<D>(ws, c, H, h), [&](int part) { fetch(next, part); });
     }
 }
 
@@ -1220,7 +1226,7 @@ static int launch_state(int T, int H, const char *ws, float *S, float *o, hipStr
     return launch_state_nw<D, 1>(T, H, ws, S, o, co, st);
 }
 
-template <int D>
+template <int D, bool KEEP>
 static int launch_chunk(int T, int H, const float *q, const float *k, const float *v,
                         const float *g, const float *beta, float qs, float *S, float *o,
                         char *ws, hipStream_t st)
@@ -1229,10 +1235,10 @@ static int launch_chunk(int T, int H, const float *q, const float *k, const floa
     const size_t lds = P1Lds<D>::FLOATS * sizeof(float);
     static bool lds_ok = false;
     int ncu = 0, rc;
-    if ((rc = allow_lds((const void *)kda_chunk_intra<D>, lds, lds_ok))) return rc;
+    if ((rc = allow_lds((const void *)kda_chunk_intra<D, KEEP>, lds, lds_ok))) return rc;
     if ((rc = cu_count(ncu))) return rc;
     const int grid = (int)(nitems < ncu ? nitems : ncu);   // one 150 KiB-LDS workgroup per CU
-    hipLaunchKernelGGL((kda_chunk_intra<D>), dim3(grid), dim3(P1_THREADS), lds, st, T, H, qs, q, k,
+    hipLaunchKernelGGL((kda_chunk_intra<D, KEEP>), dim3(grid), dim3(P1_THREADS), lds, st, T, H, qs, q, k,
                        v, g, beta, ws);
     K3_LAUNCHED();
     return launch_state<D>(T, H, ws, S, o, st);
@@ -1248,22 +1254,35 @@ struct PrefillArgs {
     char *ws;
 };
 
-template <int D, int K, int DT>
-static int launch_prefill(const PrefillArgs &a, hipStream_t st)
+template <int D, int K, int DT, bool KEEP>
+static int launch_prefill_keep(const PrefillArgs &a, hipStream_t st)
 {
     const long nitems = (long)((a.T + CH - 1) / CH) * a.H;
     const size_t lds = (P1Lds<D>::FLOATS + 3 * D * 4 + D) * sizeof(float);
     static bool lds_ok = false;
     int ncu = 0, rc;
-    if ((rc = allow_lds((const void *)kda_chunk_intra_act<D, K, DT>, lds, lds_ok))) return rc;
+    if ((rc = allow_lds((const void *)kda_chunk_intra_act<D, K, DT, KEEP>, lds, lds_ok))) return rc;
     if ((rc = cu_count(ncu))) return rc;
     const int grid = (int)(nitems < ncu ? nitems : ncu);
-    hipLaunchKernelGGL((kda_chunk_intra_act<D, K, DT>), dim3(grid), dim3(P1_THREADS), lds, st, a.T,
+    hipLaunchKernelGGL((kda_chunk_intra_act<D, K, DT, KEEP>), dim3(grid), dim3(P1_THREADS), lds, st, a.T,
                        a.H, a.qs, a.lb, a.qi, a.ki, a.vi, a.z, a.bl, a.qc, a.kc, a.vc, a.A, a.dt,
                        a.cs, a.ws);
     K3_LAUNCHED();
     // phase 2 also writes the outgoing conv history (the kernel above has read the incoming one)
     return launch_state<D>(a.T, a.H, a.ws, a.S, a.o, st, ConvOut{a.qi, a.ki, a.vi, a.cs, K, DT});
+}
+
+// The pass's workspace, chunks x heads blocks, decides where phase 1's stores go (store_ws).
+template <int D>
+static bool ws_cached(int T, int H)
+{
+    return (size_t)((T + CH - 1) / CH) * H * Ws<D>::SIZE <= WS_CACHED_BYTES;
+}
+
+template <int D, int K, int DT>
+static int launch_prefill(const PrefillArgs &a, hipStream_t st)
+{
+    return ws_cached<D>(a.T, a.H) ? launch_prefill_keep<D, K, DT, true>(a, st) : launch_prefill_keep<D, K, DT, false>(a, st);
 }
 
 template <int D, int DT>
@@ -1339,10 +1358,9 @@ extern "C" int k3hip_kda_chunk(int T, int H, int D, int chunk, const float *q, c
     for (long t0 = 0; t0 < T; t0 += pass) {
         const int Ts = (int)std::min(pass, (long)T - t0);
         const size_t r = (size_t)t0 * P;
-        const int rc = D == 128 ? launch_chunk<128>(Ts, H, q + r, k + r, v + r, g + r, beta + (size_t)t0 * H, q_scale,
-                                                    S, o + r, ws, st)
-                                : launch_chunk<64>(Ts, H, q + r, k + r, v + r, g + r, beta + (size_t)t0 * H, q_scale,
-                                                   S, o + r, ws, st);
+        auto run = [&](auto fn) { return fn(Ts, H, q + r, k + r, v + r, g + r, beta + (size_t)t0 * H, q_scale, S, o + r, ws, st); };
+        const int rc = D == 128 ? (ws_cached<128>(Ts, H) ? run(launch_chunk<128, true>) : run(launch_chunk<128, false>))
+                                : (ws_cached<64>(Ts, H) ? run(launch_chunk<64, true>) : run(launch_chunk<64, false>));
         if (rc) return rc;
     }
     return K3HIP_OK;

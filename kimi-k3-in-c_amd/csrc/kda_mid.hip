@@ -51,7 +51,7 @@ struct MidArgs {
     int n, tiles_m, tiles_n;
 };
 
-__device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+[[maybe_unused]] __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 template <int n> __device__ __forceinline__ void wait_vm()   // vmcnt(n) lgkmcnt(0)
 {
@@ -69,7 +69,7 @@ template <bool F16> __device__ __forceinline__ f32x4 mfma(const u32x4 &a, const 
 
 // bf16 pair of two floats, and the pair of what the rounding left
 __device__ __forceinline__ uint32_t pack2(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, bf16x2)); }
-__device__ __forceinline__ uint32_t pack2_rest(float a, float b, uint32_t hi)
+[[maybe_unused]] __device__ __forceinline__ uint32_t pack2_rest(float a, float b, uint32_t hi)
 {
     return pack2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
 }
