@@ -138,14 +138,10 @@ int rows_frag_pack(const uint16_t *W, int N, int K, uint16_t *Wf, hipStream_t st
 size_t gemm_rows_ws_floats(int B, int N, int K);
 int gemm_rows(int B, int N, int K, const float *x, long ldx, const uint16_t *Wf, float *C, long ldc,
               hipStream_t st, float *ws = nullptr, size_t ws_floats = 0, bool c_zeroed = false);
-// gemm_rows with C also written as bf16 hi (rows 0 .. B-1), mid (B .. 2B-1) and lo (2B .. 3B-1)
-// rows of hl (row stride ldhl; the bits of split_rows3 on C), in the same launch when the
-// product runs unsplit (otherwise split_rows3 after it, ldc = ldhl = N).
-// xw != nullptr (unsplit products only, gemm_rows_splits(N, K) == 1): the x rows are
-// RMS-normalised with weight xw and eps xeps on the way in (the rmsnorm of k3_ops.c:94-102).
-int gemm_rows_hl(int B, int N, int K, const float *x, long ldx, const uint16_t *Wf, float *C, long ldc,
-                 uint16_t *hl, long ldhl, hipStream_t st, float *ws = nullptr, size_t ws_floats = 0,
-                 const float *xw = nullptr, float xeps = 0.0f);
+// gemm_rows with the x rows RMS-normalised with weight xw and eps xeps on the way in (the
+// rmsnorm of k3_ops.c:94-102); unsplit products only (gemm_rows_splits(N, K) == 1).
+int gemm_rows_norm(int B, int N, int K, const float *x, long ldx, const uint16_t *Wf, float *C, long ldc,
+                   const float *xw, float xeps, hipStream_t st);
 // gemm_rows on S = gemm_rows_plane_count(N, K) K-ranges, the count that spreads the
 // workgroups most evenly over the CUs when N has fewer column blocks than there are CUs (1:
 // unsplit), summed in range order into C by a second launch; ws holds S B N floats.
@@ -170,7 +166,7 @@ int gemm_rows_with_part(int B, int K, const float *x, long ldx, int N1, const ui
 // the kernel from the absorb product A2 [planes B][H CW] (first KL of each head's CW columns) and
 // q [B][H][QN + CW - KL] (rope at column QN); cache [B][cap][CW] fp32 (latent = channels
 // 0..KL-1), positions 0..Tn-1; chat = softmax(scale qcat . cache^T) . latent (its position
-// ranges merged into the bf16 hi / mid / lo rows of ch3 [3B][H KL], 16-byte aligned), then
+// ranges merged into chat [B][H KL], 16-byte aligned), then
 // o [B][H VH] = (chat_h . W_UV_h^T) * sigmoid(g) with W_UV_h the rows
 // h (QN + VH) + QN .. + VH of kvb [H (QN + VH)][KL] (bf16) and g (may be nullptr) the gate
 // logits at row stride ldg; zout[0 .. zn) = 0 on the way (may be nullptr). Shapes:
@@ -181,7 +177,7 @@ bool mla_attention_supported(int H, int KL, int CW);
 size_t mla_attention_ws_bytes(int B, int H, int KL, int Tn);
 int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, int planes, const float *q,
                   int QN, const float *cache, const uint16_t *kvb, int VH, const float *g, long ldg, float *o, float *zout, size_t zn,
-                  uint16_t *ch3, void *ws, size_t ws_bytes, hipStream_t st);
+                  float *chat, void *ws, size_t ws_bytes, hipStream_t st);
 
 // One decode token of a KDA layer between its projections (kda_step.hip): K1 + K3 + K4 per
 // (head, sequence). Cin rows (stride ldc) hold q | k | v at columns 0, P, 2P and the beta

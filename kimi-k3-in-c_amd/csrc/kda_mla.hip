@@ -16,7 +16,7 @@
 // few-rows bf16 GEMM of kda_rows.hip (fp32 activations split into bf16 parts in registers,
 // each weight read once for all B; q_a, kv_a and g in one pass over their concatenated
 // weights), so activations keep fp32 accuracy. The absorption (W_UK_h^T q) is a bf16 MFMA
-// product per head on q's three split rows against a transposed copy of W_UK made at
+// product per head on q, split as it is read, against a transposed copy of W_UK made at
 // upload (mla_absorb_kernel, 5.5 us at 64 heads, B = 16, against 6.2 us for the library's
 // batched GEMM: 8.4 MB of W_UK read cold each step); the final W_UV_h is applied after the
 // attention the same way. The attention reads
@@ -31,6 +31,7 @@
 #include <algorithm>
 
 #include "kda_internal.h"
+#include "kda_split.h"
 
 struct k3hip_mla_weights {
     int E, H, QL, KL, QN, QR, VH, gate;
@@ -99,13 +100,14 @@ struct LatRow {
     int pos, B;
 };
 
-// The absorb product A2[r][h][c] = sum_k x[r][h QH + k] W_UK_h[k][c] for the M = B rows of
-// x, given as bf16 hi, mid and lo planes of M rows (row stride ldx) that add up to all 24
-// bits, and every head h: one 16 x 16 x 32 bf16 MFMA tile chain per wave (16 latent columns of
+// The absorb product A2[r][h][c] = sum_k x[r][h QH + k] W_UK_h[k][c] for the M = B rows of x
+// (q, fp32, row stride ldx), split into bf16 hi + mid + lo (all 24 bits) as they are read, and
+// every head h: one 16 x 16 x 32 bf16 MFMA tile chain per wave (16 latent columns of
 // one head, the M rows in tiles of 16, lo to hi, K-steps of 32 in order), fp32 results at
-// A2 + r ldc + h CW + c. Workgroup (x, h) takes
+// A2 + r ldc + h CW + c. (Split rows written by the q_b product cost it three scattered 2-byte
+// stores an element and this kernel a third more loads.) Workgroup (x, h) takes
 // columns 64 x .. 64 x + 63 of head h. VEC: x's rows and head offsets are 16-byte aligned
-// and QN is a multiple of 8 (QH, QN and ldx multiples of 8), so each lane's 8 K values are
+// and QN is a multiple of 8 (QH and ldx multiples of 4), so each lane's 8 K values are
 // one load or none. Workgroups (x, y) with y >= H write one latent row each.
 // KS = QNP / 32 K-steps, a template constant so that a tile's loads are
 // issued together and waited for once (with a run-time count each load waited alone: 5.9 us).
@@ -113,7 +115,7 @@ typedef __bf16 mla_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mla_f32x4 __attribute__((ext_vector_type(4)));
 template <bool VEC, int KS>
 __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, int KL, int CW,
-                                                         const uint16_t *__restrict__ x, long ldx,
+                                                         const float *__restrict__ x, long ldx,
                                                          const uint16_t *__restrict__ ukt, float *__restrict__ A2,
                                                          long ldc, int H, LatRow lr)
 {
@@ -148,29 +150,31 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, 
     for (int t = 0; t < KS; t++) bf[t] = *reinterpret_cast<const mla_bf16x8 *>(brow + 32 * t);
     for (int m0 = 0; m0 < M; m0 += 16) {
         const int r = m0 + (lane & 15);
-        const uint16_t *xr = x + (size_t)(r < M ? r : 0) * ldx + (size_t)h * QH + kq;
-        mla_bf16x8 af[3][KS];
+        const float *xr = x + (size_t)(r < M ? r : 0) * ldx + (size_t)h * QH + kq;
+        f4 xa[KS], xb[KS];
 #pragma unroll
-        for (int pt = 0; pt < 3 * KS; pt++) {
-            const int p = pt / KS, t = pt % KS;
-            const uint16_t *xp = xr + (size_t)p * M * ldx;
-            mla_bf16x8 a;
+        for (int t = 0; t < KS; t++) {
             if constexpr (VEC) {
                 // QN % 8 == 0: an 8-value group is wholly inside or past QN; a group past it (or
                 // a row past M) loads the head's first group instead and is zeroed, so every
                 // load is issued unconditionally from an address inside the row
                 const bool ok = r < M && 32 * t + kq < QN;
-                const mla_bf16x8 v = *reinterpret_cast<const mla_bf16x8 *>(xp + (ok ? 32 * t : -kq));
-                a = ok ? v : mla_bf16x8{};
+                const f4 *p = reinterpret_cast<const f4 *>(xr + (ok ? 32 * t : -kq));
+                xa[t] = p[0];
+                xb[t] = p[1];
+                if (!ok) xa[t] = xb[t] = f4(0.0f);
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    const int k = 32 * t + kq + e;
-                    a[e] = __builtin_bit_cast(__bf16, r < M && k < QN ? xp[32 * t + e] : (uint16_t)0);
+                    const float v = r < M && 32 * t + kq + e < QN ? xr[32 * t + e] : 0.0f;
+                    if (e < 4) xa[t][e] = v;
+                    else xb[t][e - 4] = v;
                 }
             }
-            af[p][t] = a;
         }
+        mla_bf16x8 af[3][KS];
+#pragma unroll
+        for (int t = 0; t < KS; t++) bsplit::split_row8(xa[t], xb[t], af[0][t], af[1][t], af[2][t]);
         mla_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int p = 2; p >= 0; p--)
@@ -186,7 +190,7 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, 
 }
 
 template <bool VEC>
-static int mla_absorb_v(int M, int H, int QH, int QN, int QNP, int KL, int CW, const uint16_t *x, long ldx,
+static int mla_absorb_v(int M, int H, int QH, int QN, int QNP, int KL, int CW, const float *x, long ldx,
                         const uint16_t *ukt, float *A2, long ldc, const LatRow &lr, hipStream_t st)
 {
     const int gx = (KL + 63) / 64;
@@ -208,12 +212,11 @@ static int mla_absorb_v(int M, int H, int QH, int QN, int QNP, int KL, int CW, c
     return K3HIP_OK;
 }
 
-// A2 = per head h, x (M rows in three planes, columns h QH .. h QH + QN - 1) . W_UK_h, via
-// mla_absorb_kernel.
-static int mla_absorb(int M, int H, int QH, int QN, int QNP, int KL, int CW, const uint16_t *x, long ldx,
+// A2 = per head h, x (M rows, columns h QH .. h QH + QN - 1) . W_UK_h, via mla_absorb_kernel.
+static int mla_absorb(int M, int H, int QH, int QN, int QNP, int KL, int CW, const float *x, long ldx,
                       const uint16_t *ukt, float *A2, long ldc, const LatRow &lr, hipStream_t st)
 {
-    if (QH % 8 == 0 && QN % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0)
+    if (QH % 4 == 0 && QN % 8 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0)
         return mla_absorb_v<true>(M, H, QH, QN, QNP, KL, CW, x, ldx, ukt, A2, ldc, lr, st);
     return mla_absorb_v<false>(M, H, QH, QN, QNP, KL, CW, x, ldx, ukt, A2, ldc, lr, st);
 }
@@ -484,7 +487,7 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     const int planes = w->ukt ? 1 : 3;
     // scratch: q_a kv_a g projections [B][ld1] | q_a normed | q | q split | absorb planes | qcat |
     //          scores or the fused attention's workspace | chat | chat split | W_UV planes (qcat,
-    //          chat and the W_UV planes only without the fused attention) | o | split-K partials
+    //          the chat split and the W_UV planes only without the fused attention) | o | split-K partials
     const int N1 = QL + CW + (w->gate ? HV : 0);
     const long ld1 = (N1 + 3) & ~3;
     // the q_a / kv_a / g product on K-ranges that spread it over every CU, summed by a second
@@ -493,10 +496,10 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     const size_t wsf = std::max({gemm_rows_ws_floats(B, N1, E), np1 > 1 ? (size_t)np1 * std::min(64, B) * N1 : 0,
                                  gemm_rows_ws_floats(B, H * QH, QL), gemm_rows_ws_floats(B, E, HV)});
     size_t sizes[] = {(size_t)B * ld1 * 4, (size_t)B * QL * 4, (size_t)B * H * QH * 4,
-                      (size_t)3 * B * H * QH * 2, (size_t)planes * B * H * CW * 4,
+                      w->ukt ? 0 : (size_t)3 * B * H * QH * 2, (size_t)planes * B * H * CW * 4,
                       fused ? 0 : (size_t)B * H * CW * 4,
                       fused ? mla_attention_ws_bytes(B, H, KL, Tn) : (size_t)B * H * Tn * 4,
-                      fused ? 0 : (size_t)B * H * KL * 4, (size_t)3 * B * H * KL * 2,
+                      (size_t)B * H * KL * 4, fused ? 0 : (size_t)3 * B * H * KL * 2,
                       fused ? 0 : (size_t)3 * B * HV * 4, (size_t)B * HV * 4, wsf * 4};
     constexpr int NB = sizeof sizes / sizeof sizes[0];
     size_t off[NB], total = 0;
@@ -529,22 +532,20 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
                            NormJob{C1 + QL, CW, KL, w->kv_a_norm, nullptr, cache}, (long)cap, pos);
         K3_LAUNCHED();
     }
-    // q, and q as bf16 hi / mid / lo rows for the absorb product, from one launch
     if (fold_norms)
-        rc = gemm_rows_hl(B, H * QH, QL, C1, ld1, (const uint16_t *)w->q_b, q, (long)H * QH, qs3, (long)H * QH, st, ws,
-                          wsf, w->q_a_norm, w->eps);
+        rc = gemm_rows_norm(B, H * QH, QL, C1, ld1, (const uint16_t *)w->q_b, q, (long)H * QH, w->q_a_norm, w->eps, st);
     else
-        rc = gemm_rows_hl(B, H * QH, QL, qn, QL, (const uint16_t *)w->q_b, q, (long)H * QH, qs3, (long)H * QH, st, ws,
-                          wsf);
+        rc = gemm_rows(B, H * QH, QL, qn, QL, (const uint16_t *)w->q_b, q, (long)H * QH, st, ws, wsf);
     if (rc) return rc;
-    // absorb: per head h, [q hi; mid; lo] (3B x QN) . W_UK_h (QN x KL)
+    // absorb: per head h, q (B x QN) . W_UK_h (QN x KL); the library GEMM takes q as split rows
     if (w->ukt) {
-        if ((rc = mla_absorb(B, H, QH, QN, w->QNP, KL, CW, qs3, (long)H * QH, (const uint16_t *)w->ukt, A2,
+        if ((rc = mla_absorb(B, H, QH, QN, w->QNP, KL, CW, q, (long)H * QH, (const uint16_t *)w->ukt, A2,
                              (long)H * CW,
                              LatRow{fold_norms ? C1 + QL : nullptr, ld1, w->kv_a_norm, w->eps, cache, (long)cap, pos, B},
                              st)))
             return rc;
     } else {
+        if ((rc = split_rows3(q, qs3, B, H * QH, st))) return rc;
         GemmDesc ga;
         ga.M = 3 * B; ga.N = KL; ga.K = QN; ga.ab_dtype = K3HIP_BF16; ga.c_dtype = K3HIP_F32; ga.b_trans = false;
         ga.lda = (long)H * QH; ga.ldb = KL; ga.ldc = (long)H * CW; ga.batch = H;
@@ -559,7 +560,7 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
         // the query rows formed inside the attention from A2 and q; the ranges merged, W_UV and
         // the output gate applied in the launch after it (kda_mla_attn.hip)
         if ((rc = mla_attention(B, H, KL, CW, Tn, cap, 1.0f / sqrtf((float)QH), A2, planes, q, QN, cache, kvb, VH, gl, ld1,
-                                o, oz ? out : nullptr, oz ? (size_t)B * E : (size_t)0, ch3, S,
+                                o, oz ? out : nullptr, oz ? (size_t)B * E : (size_t)0, chat, S,
                                 mla_attention_ws_bytes(B, H, KL, Tn), st)))
             return rc;
         return gemm_rows(B, E, HV, o, HV, (const uint16_t *)w->o, out, E, st, ws, wsf, oz);

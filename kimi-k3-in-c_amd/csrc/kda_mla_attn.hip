@@ -36,12 +36,13 @@
 //    One barrier per iteration: P of tile it and the staging of tile it + 1 are published.
 //  * Each workgroup writes its unnormalised sums with (M, l); a second kernel merges the
 //    ranges of a sequence (weights 2^(M_s - M*), the sums in a fixed order), divides by the
-//    merged sum and writes chat directly as the bf16 hi/mid/lo rows of the W_UV product.
+//    merged sum and writes chat.
 #include <math.h>
 
 #include <algorithm>
 
 #include "kda_internal.h"
+#include "kda_split.h"
 
 namespace k3kda {
 
@@ -457,13 +458,13 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 }
 
 // Block (h, b): merge the nsplit ranges of sequence b, head h, in range order; write
-// chat = sum / l as bf16 hi (row b), mid (row B + b) and lo (row 2B + b) of ch3 [3B][H KL]. Thread i covers
+// chat = sum / l, row b of chat [B][H KL]. Thread i covers
 // channels 4i .. 4i + 3 (and every 4 * blockDim further).
 __global__ __launch_bounds__(128) void mla_attn_merge_kernel(int B, int H, int KL, int nsplit,
                                                              const float *__restrict__ pctx,
                                                              const float *__restrict__ pm,
                                                              const float *__restrict__ pl,
-                                                             uint16_t *__restrict__ ch3)
+                                                             float *__restrict__ chat)
 {
     __shared__ float sw[AT_MAXSPLIT];
     __shared__ float sl;
@@ -486,27 +487,18 @@ __global__ __launch_bounds__(128) void mla_attn_merge_kernel(int B, int H, int K
     }
     __syncthreads();
     const float rl = 1.0f / sl;
-    const size_t BN = (size_t)B * H * KL;
     for (int c = 4 * tid; c < KL; c += 4 * blockDim.x) {
         f4 a = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 8
         for (int s = 0; s < nsplit; s++)
             a += sw[s] * *reinterpret_cast<const f4 *>(pctx + (((size_t)b * nsplit + s) * H + h) * KL + c);
-        const size_t i = ((size_t)b * H + h) * KL + c;
-        const float v[4] = {a.x * rl, a.y * rl, a.z * rl, a.w * rl};
-        uint16_t p[4][3];
-#pragma unroll
-        for (int e = 0; e < 4; e++) split3(v[e], p[e]);
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-            *reinterpret_cast<uint2 *>(ch3 + k * BN + i) =
-                uint2{p[0][k] | ((uint32_t)p[1][k] << 16), p[2][k] | ((uint32_t)p[3][k] << 16)};
+        *reinterpret_cast<f4 *>(chat + ((size_t)b * H + h) * KL + c) = a * rl;
     }
 }
 
 // o = (chat . W_UV_h^T) * sigmoid(g) per (head h, block of up to 16 sequences) from the merged
-// chat's bf16 hi / mid / lo rows (ch3 [3B][H KL]): all three against the bf16 weight into one fp32
-// accumulator on 16x16x32 MFMA (the products exact, the sums fp32), then the output gate
+// chat, split into bf16 hi + mid + lo on its way into LDS (half the bytes of rows split by the
+// merge, and of its stores): all three against the bf16 weight into one fp32 accumulator on 16x16x32 MFMA (the products exact, the sums fp32), then the output gate
 // sigmoid(g) (the reference's 1 / (1 + expf(-g)), src/core/k3_ops.c:105), written as fp32
 // rows of o [B][H VH] for o_proj. Replaces a head-batched W_UV GEMM and a gate kernel (two
 // launches and the GEMM's two fp32 output planes). W_UV_h = rows h (QN + VH) + QN .. + VH of
@@ -515,7 +507,7 @@ __global__ __launch_bounds__(128) void mla_attn_merge_kernel(int B, int H, int K
 constexpr int AO_NT = 512;                 // 8 waves, one 16-column tile of o each (VH <= 128)
 constexpr int AO_KP = 32 * 16 + 8;         // LDS row pitch (bf16): 16 bytes of skew per row
 __global__ __launch_bounds__(AO_NT) void mla_attn_out_kernel(int B, int H, int KL, int QN, int VH,
-                                                            const uint16_t *__restrict__ ch3,
+                                                            const float *__restrict__ chat,
                                                             const uint16_t *__restrict__ kvb,
                                                             const float *__restrict__ g, long ldg,
                                                             float *__restrict__ o, float *__restrict__ zout, size_t zn)
@@ -543,18 +535,20 @@ __global__ __launch_bounds__(AO_NT) void mla_attn_out_kernel(int B, int H, int K
 #pragma unroll
         for (int e = 0; e < 4; e++)
             if (4 * kq + e < nb) gv[e] = g[(size_t)(b0 + 4 * kq + e) * ldg + (size_t)h * VH + n];
-    // the block's chat rows (all three parts) into LDS, 8 bf16 per thread and pass; rows past nb and
+    // the block's chat rows into LDS, 8 values per thread and pass, split; rows past nb and
     // channels past KL are zero
-    const size_t BN = (size_t)B * H * KL;
     for (int it = tid; it < 16 * (KLr / 8); it += AO_NT) {
         const int r = it / (KLr / 8), c = 8 * (it % (KLr / 8));
-        uint4 v[3];
-        const size_t i = ((size_t)(b0 + r) * H + h) * KL + c;
+        f4 u = 0.0f, v = 0.0f;
+        if (r < nb && c < KL) {
+            const f4 *p = reinterpret_cast<const f4 *>(chat + ((size_t)(b0 + r) * H + h) * KL + c);
+            u = p[0];
+            v = p[1];
+        }
+        bf16x8 part[3];
+        bsplit::split_row8(u, v, part[0], part[1], part[2]);
 #pragma unroll
-        for (int p = 0; p < 3; p++)
-            v[p] = r < nb && c < KL ? *reinterpret_cast<const uint4 *>(ch3 + p * BN + i) : uint4{0, 0, 0, 0};
-#pragma unroll
-        for (int p = 0; p < 3; p++) *reinterpret_cast<uint4 *>(chs[p] + r * AO_KP + c) = v[p];
+        for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8 *>(chs[p] + r * AO_KP + c) = part[p];
     }
     if (zout) {
         const size_t nwg = (size_t)gridDim.x * gridDim.y, id = (size_t)blockIdx.y * gridDim.x + h;
@@ -640,7 +634,7 @@ bool mla_attention_supported(int H, int KL, int CW)
 
 int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, int planes, const float *q,
                   int QN, const float *cache, const uint16_t *kvb, int VH, const float *gate, long ldg, float *o, float *zout, size_t zn,
-                  uint16_t *ch3, void *ws, size_t ws_bytes, hipStream_t st)
+                  float *chat, void *ws, size_t ws_bytes, hipStream_t st)
 {
     AtGeom g;
     if (!at_geom(H, KL, CW, g))
@@ -650,7 +644,7 @@ int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, co
     const size_t need = mla_attention_ws_bytes(B, H, KL, Tn);
     const int QH = QN + (CW - KL);
     if (!ws || ws_bytes < need || ((uintptr_t)ws & 255) || ((uintptr_t)cache & 15) || ((uintptr_t)A2 & 15) ||
-        ((uintptr_t)q & 15) || (QN & 3) || (KL & 7) || ((uintptr_t)kvb & 15) || ((uintptr_t)ch3 & 15) ||
+        ((uintptr_t)q & 15) || (QN & 3) || (KL & 7) || ((uintptr_t)kvb & 15) || ((uintptr_t)chat & 15) ||
         VH < 1 || VH > 16 * (AO_NT / 64))
         K3_FAIL(K3HIP_EINVAL, "mla attention: workspace %zu < %zu bytes, or a misaligned buffer", ws_bytes, need);
     const AtQ qs{A2, q, planes, B, QN, QH};
@@ -670,9 +664,9 @@ int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, co
     void *args[] = {&g, &Tn, &cap, (void *)&nsplit, &scale2, (void *)&qs, (void *)&cache, &pctx, &pm, &pl};
     K3_HIP(hipLaunchKernel(kern, dim3(nsplit, B, groups), dim3(AT_NT), args, AT_LDS, st));
     K3_LAUNCHED();
-    hipLaunchKernelGGL(mla_attn_merge_kernel, dim3(H, B), dim3(128), 0, st, B, H, KL, nsplit, pctx, pm, pl, ch3);
+    hipLaunchKernelGGL(mla_attn_merge_kernel, dim3(H, B), dim3(128), 0, st, B, H, KL, nsplit, pctx, pm, pl, chat);
     K3_LAUNCHED();
-    hipLaunchKernelGGL(mla_attn_out_kernel, dim3(H, (B + 15) / 16), dim3(AO_NT), 0, st, B, H, KL, QN, VH, ch3, kvb,
+    hipLaunchKernelGGL(mla_attn_out_kernel, dim3(H, (B + 15) / 16), dim3(AO_NT), 0, st, B, H, KL, QN, VH, chat, kvb,
                        gate, ldg, o, zout, zn);
     K3_LAUNCHED();
     return K3HIP_OK;

@@ -71,10 +71,6 @@ struct RowsJob {
     const uint16_t *Wf;
     float *P;
     long ldp, split_stride;
-    // unsplit products only: C also as bf16 hi (row m), mid and lo (each a plane hlplane on)
-    // rows of stride ldhl, x = hi + mid + lo, for a following product on split rows (nullptr: none)
-    uint16_t *hl = nullptr;
-    long ldhl = 0, hlplane = 0;
 };
 
 // Block (nb, s) of a job: column groups 4 nb .. 4 nb + 3, K-steps [s tchunk, min(KT, (s + 1)
@@ -237,12 +233,6 @@ __global__ __launch_bounds__(64 * RT_WAVES, MT == 4 ? 2 : 4) void rows_gemm_kern
                     unsafeAtomicAdd(&out[(size_t)m * ldp + n], t[e]);
                 } else {
                     out[(size_t)m * ldp + n] = t[e];
-                    if (jb.hl) {
-                        uint16_t h3[3];
-                        split3(t[e], h3);
-#pragma unroll
-                        for (int p = 0; p < 3; p++) jb.hl[(size_t)p * jb.hlplane + (size_t)m * jb.ldhl + n] = h3[p];
-                    }
                 }
             }
         }
@@ -435,28 +425,19 @@ int gemm_rows_with_part(int B, int K, const float *x, long ldx, int N1, const ui
     return K3HIP_OK;
 }
 
-int gemm_rows_hl(int B, int N, int K, const float *x, long ldx, const uint16_t *Wf, float *C, long ldc,
-                 uint16_t *hl, long ldhl, hipStream_t st, float *ws, size_t ws_floats, const float *xw, float xeps)
+int gemm_rows_norm(int B, int N, int K, const float *x, long ldx, const uint16_t *Wf, float *C, long ldc,
+                   const float *xw, float xeps, hipStream_t st)
 {
     if (B <= 0 || N <= 0 || K <= 0) return K3HIP_OK;
     const RowsPlan pl = rows_plan(N, K);
-    if (xw && (pl.S != 1 || (((uintptr_t)xw) & 15)))
-        K3_FAIL(K3HIP_EUNSUPPORTED, "gemm_rows_hl: the normalised input needs an unsplit product and 16-byte aligned weights");
-    if (pl.S != 1) {   // the split rows from the reduced product
-        int rc = gemm_rows(B, N, K, x, ldx, Wf, C, ldc, st, ws, ws_floats);
-        if (rc) return rc;
-        if (ldhl != N || ldc != N) K3_FAIL(K3HIP_EINVAL, "gemm_rows_hl: a split-K product needs ldc = ldhl = N");
-        return split_rows3(C, hl, B, N, st);
-    }
+    if (pl.S != 1 || (((uintptr_t)xw) & 15))
+        K3_FAIL(K3HIP_EUNSUPPORTED, "gemm_rows_norm: needs an unsplit product and 16-byte aligned weights");
     if ((K & 7) || (ldx & 3) || (((uintptr_t)x | (uintptr_t)Wf) & 15))
-        K3_FAIL(K3HIP_EINVAL, "gemm_rows_hl: K=%d ldx=%ld need multiples of 8 / 4 and 16-byte aligned x, W", K, ldx);
+        K3_FAIL(K3HIP_EINVAL, "gemm_rows_norm: K=%d ldx=%ld need multiples of 8 / 4 and 16-byte aligned x, W", K, ldx);
     const RowsJob none{1, 1, 0, 1, Wf, C, 0, 0};   // no blocks
     for (int b0 = 0; b0 < B; b0 += 64) {
         const int bb = std::min(64, B - b0);
-        RowsJob j = rows_job(N, pl.tchunk, 1, Wf, C + (size_t)b0 * ldc, ldc, 0);
-        j.hl = hl + (size_t)b0 * ldhl;
-        j.ldhl = ldhl;
-        j.hlplane = (long)B * ldhl;
+        const RowsJob j = rows_job(N, pl.tchunk, 1, Wf, C + (size_t)b0 * ldc, ldc, 0);
         int rc = launch_jobs_b(bb, K, x + (size_t)b0 * ldx, ldx, j, none, st, xw, xeps);
         if (rc) return rc;
     }

@@ -2,7 +2,8 @@
 """The MLA attention's head groups and head tiles (csrc/kda_mla_attn.hip) against the oracle at
 the decode bar (rtol 1e-4, atol 1e-4 rms): head counts on both sides of each 16-head tile and
 64-head group, groups of unequal size, contexts of one tile, several ranges and a ragged last
-tile; and a latent wider than the one-pass kernel holds (the batched GEMM form)."""
+tile; and a latent wider than the one-pass kernel holds (the batched GEMM form, at a context for
+each of its three softmax variants)."""
 from __future__ import annotations
 
 import numpy as np
@@ -18,7 +19,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("H,kvl,qr,B,start,gate", [
     (16, 512, 64, 2, 150, 1), (17, 64, 16, 3, 33, 0), (33, 512, 64, 1, 20, 1), (48, 64, 16, 25, 40, 1),
     (65, 512, 64, 2, 150, 1), (96, 512, 64, 3, 47, 1), (96, 32, 8, 17, 5, 0), (128, 64, 16, 2, 300, 1),
-    (130, 48, 12, 1, 31, 1), (8, 528, 16, 2, 30, 1)])
+    (130, 48, 12, 1, 31, 1), (8, 528, 16, 2, 30, 1),
+    (4, 528, 16, 1, 2100, 1), (4, 528, 16, 1, 8300, 1)])
 def test_mla_head_groups_vs_oracle(gpu, H, kvl, qr, B, start, gate):
     """`start` cached positions written to both caches, then three steps."""
     import torch
