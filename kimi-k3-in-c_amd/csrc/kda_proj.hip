@@ -12,7 +12,7 @@
 //  * T <= 4 (fp32 weights: T <= 2), proj_gemv_kernel: a wave owns R rows of W and every token,
 //    8 consecutive inputs per lane (a 16-byte load of bf16), double FMAs on the vector unit, a
 //    butterfly over the lanes. Bound by reading W: one token of a bf16 layer of hidden 4096
-//    and 32 x 128 heads streams its 136 MB of q, k, v, g, f_a and b in 27.6 us (4.9 TB/s); one
+//    and 32 x 128 heads streams its 136 MB of q, k, v, g, f_a and b in about 25 us (the call 390 -> 43 us); one
 //    row a wave, one element a lane and eight token accumulators whatever T is took 46 us for
 //    each 34 MB matrix (0.7 TB/s).
 //  * more tokens, proj_mfma_kernel: v_mfma_f64_16x16x4_f64 tiles of 16 rows x 16 tokens, four
@@ -213,6 +213,8 @@ __global__ __launch_bounds__(64 * PJ_WAVES) void proj_gemv_kernel(const ProjArgs
     const int nb = (in + 511) / 512;
     int i = 0;
     for (; i + U <= nb; i += U) blocks(std::integral_constant<int, U>{}, 512 * i + 8 * lane);
+    if constexpr (U > 2)
+        for (; i + 2 <= nb; i += 2) blocks(std::integral_constant<int, 2>{}, 512 * i + 8 * lane);
     for (; i < nb; i++) blocks(std::integral_constant<int, 1>{}, 512 * i + 8 * lane);
 #pragma unroll
     for (int r = 0; r < R; r++)
@@ -324,13 +326,19 @@ int launch(ProjArgs &a, int T, int in, long rows, const float *x, hipStream_t st
 {
     if (T <= (WDT == K3_WF32 ? PJ_GEMV_T_F32 : PJ_GEMV_T)) {
         // Two rows a wave read x half as often, but need twice the rows to fill the GPU:
-        // they run from 8192 rows on (32 waves of two rows per CU); below, one row a wave.
+        // they run from 8192 rows on (32 waves of two rows per CU); below, one row a wave. (Four
+        // rows: the token of the bf16 layer above 46.3 us against 43.1, fp32 120 against 81.)
+        // One bf16 token keeps four blocks of 512 inputs in flight, its weights being one load
+        // each (43.1 us, two blocks 45.7); fp32, twice the loads, two (80.8 against 85.5).
         const int R = rows >= 8192 ? 2 : 1;
         const unsigned blocks = (unsigned)((deal(a, R) + PJ_WAVES - 1) / PJ_WAVES);
 #define K3_GEMV(TB, RR, UU) \
     hipLaunchKernelGGL((proj_gemv_kernel<WDT, TB, RR, UU, VEC>), dim3(blocks), dim3(64 * PJ_WAVES), 0, st, a, T, in, x)
         if (R == 2) {
-            if (T == 1) K3_GEMV(1, 2, 2);
+            if (T == 1) {
+                if constexpr (WDT == K3_WBF16) K3_GEMV(1, 2, 4);
+                else K3_GEMV(1, 2, 2);
+            }
             else if (T == 2) K3_GEMV(2, 2, 2);
             else if constexpr (WDT != K3_WF32) K3_GEMV(4, 2, 1);
         } else {
