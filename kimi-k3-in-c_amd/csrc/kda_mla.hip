@@ -17,8 +17,9 @@
 // each weight read once for all B; q_a, kv_a and g in one pass over their concatenated
 // weights), so activations keep fp32 accuracy. The absorption (W_UK_h^T q) is a bf16 MFMA
 // product per head on q, split as it is read, against a transposed copy of W_UK made at
-// upload (mla_absorb_kernel, 5.5 us at 64 heads, B = 16, against 6.2 us for the library's
-// batched GEMM: 8.4 MB of W_UK read cold each step); the final W_UV_h is applied after the
+// upload (mla_absorb_kernel, 6.9 us at 64 heads, B = 16, with all of q's 24 bits and the new
+// latent row; the library's batched GEMM took 6.2 us on two split rows: 8.4 MB of W_UK read cold each
+// step); the final W_UV_h is applied after the
 // attention the same way. The attention reads
 // the cache once where the shape fits the fused kernel (kda_mla_attn.hip: split-bf16 MFMA
 // scores, online softmax with the reference's scale (nope+rope)^-0.5, split-bf16 weighted

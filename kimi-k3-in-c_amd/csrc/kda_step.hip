@@ -24,7 +24,8 @@
 // kda_epilogue2_kernel except for the row's sum of squares: fp32 per-lane squares added
 // across the half-wave by DPP in fp32 (the epilogue kernel adds the lanes in double; for a
 // 128-channel head the two differ by a few 1e-7 relative) and the hardware reciprocal
-// square root; hardware sigmoid. The output-gate logits may arrive as split-K partial planes of the gate
+// square root (step_exact, the full-accuracy layer's one-token call, keeps the epilogue kernel's
+// double sum and root); hardware sigmoid. The output-gate logits may arrive as split-K partial planes of the gate
 // projection; they are added in plane order, which is what the split-K reduction does.
 //
 // The core form (k3hip_kda_decode_step) takes the decay logits z and the conv inputs as
