@@ -117,6 +117,14 @@ void ws_drop(WsPool &P, size_t i)
     P.blocks.erase(P.blocks.begin() + (long)i);
 }
 
+// Event queries are kept out of the rules of a capture that another stream or thread may have
+// open in its global mode.
+struct RelaxedCapture {
+    hipStreamCaptureMode m = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&m); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&m); }
+};
+
 // A kept block of at least `bytes` for a call on st, or nullptr: take a plain allocation.
 WsBlock *ws_take(size_t bytes, hipStream_t st)
 {
@@ -139,6 +147,7 @@ WsBlock *ws_take(size_t bytes, hipStream_t st)
     if (dev < 0 || dev >= 64 || size > WS_KEEP_BYTES) return nullptr;
     std::lock_guard<std::mutex> lock(P.mu);
     if (P.handles <= 0) return nullptr;
+    RelaxedCapture relaxed;
     WsBlock *best = nullptr;
     for (WsBlock *k : P.blocks) {
         if (k->busy || k->dev != dev || k->size < bytes || (best && best->size <= k->size)) continue;
