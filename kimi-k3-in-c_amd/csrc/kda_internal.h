@@ -57,23 +57,23 @@ int mm_splitk(int M, int N, int K, int splits, int ab, const void *A, long lda, 
               hipStream_t st);
 
 // Several weights over the same rows in one launch (kda_mid.hip): C_s[M][rows_s] = A[M][K] .
-// B_s[rows_s][K]^T, fp32 accumulation, B_s row-major with K-contiguous rows. A: 16-bit rows
-// (bf16, or fp16 against fp16 weights with f16), or fp32 rows split into bf16 hi + lo. Columns from `cols` on (0: none) go to C1. out: K3HIP_F32, or K3HIP_BF16
-// with f16. Needs mid_supported and 16-byte aligned weights.
+// B_s[rows_s][K]^T, fp32 accumulation, bf16 B_s with K-contiguous rows. A: bf16 rows, or fp32
+// rows split into bf16 hi + lo. Columns from `cols` on (0: none) go to C1. Needs mid_supported
+// and 16-byte aligned weights.
 constexpr int MID_SEGS = 5;
 enum { MID_A_16 = 0, MID_A_SPLIT = 1 };
 struct MidSeg {
     const void *B;
-    void *C;
+    float *C;
     long ldc;
     int rows;
     int cols = 0;
-    void *C1 = nullptr;
+    float *C1 = nullptr;
     long ldc1 = 0;
     bool vec = false;   // set by mid()
 };
 bool mid_supported(int K, const void *A, long lda, bool a_fp32);
-int mid(int M, int K, int a_mode, const void *A, long lda, const MidSeg *segs, int n, bool f16, int out, hipStream_t st);
+int mid(int M, int K, int a_mode, const void *A, long lda, const MidSeg *segs, int n, hipStream_t st);
 
 // K4 with y written as a bf16 hi/lo pair into y2 [T][2P] (hi columns 0..P-1, lo P..2P-1),
 // for an o_proj GEMM with K = 2P against [W_o | W_o]. D = 64 / 128, 16-byte aligned.

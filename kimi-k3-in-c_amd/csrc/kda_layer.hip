@@ -554,7 +554,7 @@ extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out
         if (!mfma) return proj(T, nin, nout, in, W, w->wdt, y, st);
         if (!big) {
             const MidSeg s{W, y, nout, nout};
-            return mid(T, nin, MID_A_SPLIT, in, nin, &s, 1, false, K3HIP_F32, st);
+            return mid(T, nin, MID_A_SPLIT, in, nin, &s, 1, st);
         }
         int r = mm(2 * T, nout, nin, K3HIP_BF16, xs, nin, W, nin, C2, K3HIP_F32, nout, st);
         return r ? r : pair_add(C2, y, T, nout, st);
@@ -572,7 +572,7 @@ extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out
     } else if (mfma) {
         const MidSeg in[5] = {{w->q, qp, iP, iP}, {w->k, kp, iP, iP}, {w->v, vp, iP, iP}, {w->g, gl, iP, iP},
                               {w->f_a, fa, D, D + H, D, bl, H}};
-        if ((rc = mid(T, E, MID_A_SPLIT, x, E, in, 5, false, K3HIP_F32, st))) return rc;
+        if ((rc = mid(T, E, MID_A_SPLIT, x, E, in, 5, st))) return rc;
     } else {
         const ProjSeg in[6] = {{w->q, qp, iP}, {w->k, kp, iP}, {w->v, vp, iP}, {w->g, gl, iP}, {w->f_a, fa, D}, {w->b, bl, H}};
         if ((rc = proj_multi(T, E, in, 6, x, w->wdt, st))) return rc;
@@ -731,12 +731,6 @@ extern "C" int k3hip_set_projection_gemm(int impl)
     return K3HIP_OK;
 }
 
-// Products of the input projections (T x their rows x hidden) up to which the short form of the
-// prefill runs: against the library's launches, hidden 4096 and 32 x 128 heads T = 330 (22e9)
-// 185 -> 149 us, T = 420 (28e9) 200 | 207; hidden 4096 and 16 x 64 heads T = 1400 (24e9) 207 ->
-// 152; hidden 2048 and 48 x 128 heads T = 450 (23e9) 222 -> 192, T = 700 (36e9) 272 | 280.
-constexpr double MID_PREFILL_MACS = 24e9;
-
 extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *out, int out_dtype,
                                        const void *x, int x_dtype, float *state, void *stream)
 {
@@ -762,7 +756,7 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
     // The 4096-deep projections are plain GEMMs and run on hipBLASLt by default: the
     // hand-written MFMA GEMM (kda_mm.hip, k3hip_proj_gemm) matches it within 1-2% on the
     // 4096-wide ones but not on q/k/v, whose fp32 output stores keep it at ~0.93x; the 256-deep
-    // z product runs on the hand-written kernel either way (faster there).
+    // z product runs on hand-written kernels either way (faster there).
     // k3hip_set_projection_gemm(K3HIP_GEMM_HANDWRITTEN) selects the hand-written kernels for
     // every projection (`own`).
     // The hand-written kernel needs hidden % 64 == 0 and a 16-byte aligned bf16 x (an fp32 x is
@@ -772,17 +766,15 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
                      mm_supported(E, E, E) && (x_dtype == K3HIP_F32 || ((uintptr_t)x & 15) == 0);
     int ncu = 256, rc;
     if ((rc = cu_count(ncu))) return rc;
-    // Short prefills: all input projections in one launch, z and o_proj in one each (kda_mid.hip).
-    const bool sh = !own && (double)T * (4.0 * P + D + H) * E <= MID_PREFILL_MACS && mid_supported(E, x_dtype == K3HIP_F32 ? nullptr : x, E, false);
     const int fab_s = own ? mm_splits(T, D + H, E, ncu) : 1;
     // scratch, 256-byte aligned pieces:
     //   0 x bf16 | 1 q k v projections fp32 | 2 f_a and b fp32 (split-K planes) | 3 f_a hi/lo bf16 |
     //   4 z fp32 | 5 b logits | 6 o fp32 | 7 gate fp16 | 8 y fp16 | 9 zero state | 10 chunk workspace |
-    //   11 fp32 o_proj result (library path with a bf16 out) | 12 gate fp32 (short prefills)
+    //   11 fp32 o_proj result (fallback path with a bf16 out)
     size_t sizes[] = {x_dtype == K3HIP_F32 ? (size_t)T * E * 2 : 0, 3 * TP * 4, (size_t)fab_s * T * (D + H) * 4,
                       (size_t)T * D * 4, TP * 4, (size_t)T * H * 4, TP * 4, TP * 2, TP * 2,
                       state ? 0 : (size_t)H * D * D * 4, wsb,
-                      (!own && !sh && out_dtype == K3HIP_BF16) ? (size_t)T * E * 4 : 0, sh ? TP * 4 : 0};
+                      (!own && out_dtype == K3HIP_BF16) ? (size_t)T * E * 4 : 0};
     constexpr int NB = sizeof sizes / sizeof sizes[0];
     size_t off[NB], total = 0;
     for (int i = 0; i < NB; i++) {
@@ -820,16 +812,7 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
     //   2e-3 bar): q, k, v as one GEMM over their consecutive weight rows, its three column
     //   groups written to three [T][P] arrays; f_a and b as one split-K GEMM whose reduction
     //   writes f_a as a bf16 hi/lo pair for z = [f_a_hi | f_a_lo] [W_fb | W_fb]^T (fp32 accuracy)
-    const int iP = (int)P;
-    float *gl = sh ? (float *)(base + off[12]) : z;   // the library path's gate takes z's place, consumed by then
-    if (sh) {
-        // f_a stays fp32; the z product splits it as it reads it
-        const MidSeg in[5] = {{w->q, qp, iP, iP}, {w->k, kp, iP, iP}, {w->v, vp, iP, iP}, {w->g, gl, iP, iP},
-                              {w->f_a, fa, D, D + H, D, bl, H}};
-        const MidSeg zs{w->f_b, z, iP, iP};
-        if ((rc = mid(T, E, MID_A_16, xb, E, in, 5, false, K3HIP_F32, st))) return rc;
-        if ((rc = mid(T, D, MID_A_SPLIT, fa, D, &zs, 1, false, K3HIP_F32, st))) return rc;
-    } else if (own) {
+    if (own) {
         if ((rc = mm(T, 3 * (int)P, E, K3HIP_BF16, xb, E, wq, E, qp, K3HIP_F32, (long)P, st, (int)P, (long)TP)))
             return rc;
         if ((rc = mm_splitk(T, D + H, E, fab_s, K3HIP_BF16, xb, E, w->f_a, E, fa, st))) return rc;
@@ -847,7 +830,14 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
         hipLaunchKernelGGL(split_fa_b_kernel, dim3(grid_for((size_t)T * (D + H))), dim3(256), 0, st, fa,
                            fa2, bl, D, H, (size_t)T * (D + H));
         K3_LAUNCHED();
-        if (mm_supported(2 * D, 2 * D, 2 * D))
+        // z: the tiles of kda_mid.hip while the 256 x 256 ones of kda_mm.hip would leave half the CUs
+        // idle (the same bits, both sum K in order into one accumulator). T = 333, 16 x 128 heads (16
+        // tiles): 10.6 -> 7.3 us back to back; T = 2048, 32 x 128 (128 tiles): 15.3 -> 12.7; T = 1400,
+        // 48 x 128 (144) 14.7 | 17.2; T = 8192, 32 x 128 (512) 37.3 | 41.4.
+        if (2L * ((T + 255) / 256) * (((long)P + 255) / 256) <= ncu) {
+            const MidSeg zs{w->f_b2, z, (long)P, (int)P};
+            rc = mid(T, 2 * D, MID_A_16, fa2, 2 * D, &zs, 1, st);
+        } else if (mm_supported(2 * D, 2 * D, 2 * D))
             rc = mm(T, (int)P, 2 * D, K3HIP_BF16, fa2, 2 * D, w->f_b2, 2 * D, z, K3HIP_F32, (long)P, st);
         else
             rc = gemm_bf16(T, (int)P, 2 * D, fa2, w->f_b2, z, K3HIP_F32, st);
@@ -867,14 +857,11 @@ extern "C" int k3hip_kda_layer_prefill(const k3hip_kda_weights *w, int T, void *
         // 9 o_proj on fp16 MFMA against the fp16 copy of W_o
         return mm(T, E, (int)P, K3_DT_F16, y16, (long)P, w->o16, (long)P, out, out_dtype, E, st);
     }
-    // hipBLASLt has no bf16-in, fp16-out algorithm: this path keeps fp32 gate logits, as the
-    // short one does
-    if (!sh && (rc = gemm_bf16(T, iP, E, xb, w->g, gl, K3HIP_F32, st))) return rc;
+    // hipBLASLt has no bf16-in, fp16-out algorithm: this path keeps fp32 gate logits (z is
+    // consumed by now)
+    float *gl = z;
+    if ((rc = gemm_bf16(T, (int)P, E, xb, w->g, gl, K3HIP_F32, st))) return rc;
     if ((rc = epilogue_split(T, H, D, w->rms_eps, o, gl, K3HIP_F32, w->o_norm, y16, st, true))) return rc;
-    if (sh) {
-        const MidSeg os{w->o16, out, E, E};
-        return mid(T, iP, MID_A_16, y16, iP, &os, 1, true, out_dtype, st);
-    }
     if (out_dtype == K3HIP_F32) return gemm_f16(T, E, (int)P, y16, w->o16, out, K3HIP_F32, st);
     float *o32 = (float *)(base + off[11]);
     if ((rc = gemm_f16(T, E, (int)P, y16, w->o16, o32, K3HIP_F32, st))) return rc;

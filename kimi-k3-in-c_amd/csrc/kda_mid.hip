@@ -1,22 +1,23 @@
 // SPDX-License-Identifier: Apache-2.0
-// kda_mid.hip - the layer's projections for short and middle-sized prefills: several weights
-// over the same rows in one launch, for gfx950.
+// kda_mid.hip - products of short and middle-sized prefills: several weights over the same rows
+// in one launch, for gfx950.
 //
 // Replaces the reference's per-token k3_mmw calls (include/k3/k3.h:290-296 ->
 // k3_matmul_bf16, src/core/k3_ops.c:1122-1227; call sites :877-886, :946-948):
 //   C_s[M][rows_s] = A[M][K] . B_s[rows_s][K]^T     for up to MID_SEGS weights B_s
 // with fp32 accumulation. A is one of
-//   16-bit rows (bf16, or fp16 against fp16 weights),
+//   bf16 rows (the z product of the bf16 prefill, on f_a's split rows),
 //   fp32 rows split into bf16 hi + lo, both against the bf16 weight (fp32 accuracy: x = hi + lo
-//   to 2.5e-6 relative rms), which needs no split rows or second half of the result in memory.
+//   to 2.5e-6 relative rms), which needs no split rows or second half of the result in memory
+//   (the full-accuracy layer).
 //
 // The 256 x 256 tiles of kda_mm.hip leave most of the GPU idle here (333 tokens of a hidden
 // 2048, 16 x 128 layer: 2 x 33 tiles over 256 CUs, and 16 for z), and a launch per weight
 // costs more than its products. Tiles of 64 rows x 128 columns (64 x 64 where those would not
-// give every CU one, 128 x 128 where those do), four waves in 2 x 2, K in steps of 64. Weights
-// and 16-bit rows come by direct-to-LDS buffer loads into 2, 3 or 5 buffers, each requested
+// give every CU one, 128 x 128 for bf16 rows where those do), four waves in 2 x 2, K in steps of
+// 64. Weights and bf16 rows come by direct-to-LDS buffer loads into 2, 3 or 5 buffers, each requested
 // 1, 2 or 4 steps before it is read; fp32 rows go through registers one step ahead and are
-// split as they are put in LDS (two buffers). 64-112 KiB of LDS; where two workgroups share a
+// split as they are put in LDS (two buffers). 64-80 KiB of LDS; where two workgroups share a
 // CU, one's barrier and load waits hide behind the other's products. Rows are 128 bytes, the
 // 16-byte chunk index XORed with (row & 7) ^ ((row >> 3) & 1): 16-lane fragment reads fall on
 // distinct banks. The weight is the MFMA's first operand, so a lane ends with four adjacent
@@ -25,9 +26,7 @@
 //
 // Bound by the chain of a K-step (barrier, LDS reads, products) with 1 to 2 waves per SIMD, then
 // by LDS bandwidth (a 64 x 128 step reads 192 bytes per clock at the MFMAs' full rate, the LDS
-// gives 128). 333 tokens, hidden 2048, 16 x 128 heads (11.4 GMAC): the five input products 23.6 us
-// in one launch (0.97 PFLOP/s) against 45 in the library's three and a split; z 5.1 us against
-// 12.8; o_proj 12.2, bf16 results included, against 15.5; the layer 108 -> 85-87 us.
+// gives 128).
 #include "kda_internal.h"
 
 #include <algorithm>
@@ -38,7 +37,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
@@ -59,12 +57,9 @@ template <int n> __device__ __forceinline__ void wait_vm()   // vmcnt(n) lgkmcnt
     __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4));
 }
 
-template <bool F16> __device__ __forceinline__ f32x4 mfma(const u32x4 &a, const u32x4 &b, const f32x4 &c)
+[[maybe_unused]] __device__ __forceinline__ f32x4 mfma(const u32x4 &a, const u32x4 &b, const f32x4 &c)
 {
-    if constexpr (F16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 // bf16 pair of two floats, and the pair of what the rounding left
@@ -74,7 +69,7 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) { return __builtin_b
     return pack2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
 }
 
-template <int AM, int BM, int BN, int NBUF, bool F16, typename OUT>
+template <int AM, int BM, int BN, int NBUF>
 __global__ __launch_bounds__(NT, 2) void mid_kernel(const MidArgs ar, int M, int K, const void *__restrict__ Av, long lda)
 {
 #ifdef __HIP_DEVICE_COMPILE__   // the host pass, which only needs the stub, drops it over the 16-byte LDS loads
@@ -206,7 +201,7 @@ __global__ __launch_bounds__(NT, 2) void mid_kernel(const MidArgs ar, int M, int
 #pragma unroll
                 for (int i = 0; i < TI; i++)
 #pragma unroll
-                    for (int j = 0; j < TJ; j++) acc[i][j] = mfma<F16>(b[s][j], a[s][p][i], acc[i][j]);
+                    for (int j = 0; j < TJ; j++) acc[i][j] = mfma(b[s][j], a[s][p][i], acc[i][j]);
         if constexpr (AM != MID_A_16) put_a32(ks + 1);
     }
     wait_vm<0>();   // no load may still be writing this workgroup's LDS when it ends
@@ -222,28 +217,21 @@ __global__ __launch_bounds__(NT, 2) void mid_kernel(const MidArgs ar, int M, int
             const int n = n0 + wn * (BN / 2) + 16 * j + 4 * kq;
             const f32x4 v = acc[i][j];
             if (sg.vec && n + 4 <= sg.cols) {
-                OUT *p = reinterpret_cast<OUT *>(sg.C) + (long)m * sg.ldc + n;
-                if constexpr (sizeof(OUT) == 4)
-                    *reinterpret_cast<f32x4 *>(p) = v;
-                else
-                    *reinterpret_cast<uint2 *>(p) = uint2{(uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                                                          (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16)};
+                *reinterpret_cast<f32x4 *>(sg.C + (long)m * sg.ldc + n) = v;
                 continue;
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 if (n + e >= sg.rows) continue;
-                OUT *p = n + e < sg.cols ? reinterpret_cast<OUT *>(sg.C) + (long)m * sg.ldc + n + e
-                                         : reinterpret_cast<OUT *>(sg.C1) + (long)m * sg.ldc1 + (n + e - sg.cols);
-                if constexpr (sizeof(OUT) == 4) *p = v[e];
-                else *p = f2bf(v[e]);
+                float *p = n + e < sg.cols ? sg.C + (long)m * sg.ldc + n + e : sg.C1 + (long)m * sg.ldc1 + (n + e - sg.cols);
+                *p = v[e];
             }
         }
     }
 #endif
 }
 
-template <int AM, int BM, int BN, int NBUF, bool F16, typename OUT>
+template <int AM, int BM, int BN, int NBUF>
 int launch_tile(MidArgs &a, int M, int K, const void *A, long lda, hipStream_t st)
 {
     constexpr int lds = NBUF * BN * ROW + (AM == MID_A_16 ? NBUF : 4) * BM * ROW;
@@ -255,14 +243,14 @@ int launch_tile(MidArgs &a, int M, int K, const void *A, long lda, hipStream_t s
     }
     const long grid = (long)((a.tiles_n + 7) / 8) * 8 * a.tiles_m;
     if (grid > 0x7fffffffL) K3_FAIL(K3HIP_EUNSUPPORTED, "mid: %d rows need too many workgroups", M);
-    K3_HIP(hipFuncSetAttribute((const void *)mid_kernel<AM, BM, BN, NBUF, F16, OUT>,
+    K3_HIP(hipFuncSetAttribute((const void *)mid_kernel<AM, BM, BN, NBUF>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    hipLaunchKernelGGL((mid_kernel<AM, BM, BN, NBUF, F16, OUT>), dim3((unsigned)grid), dim3(NT), lds, st, a, M, K, A, lda);
+    hipLaunchKernelGGL((mid_kernel<AM, BM, BN, NBUF>), dim3((unsigned)grid), dim3(NT), lds, st, a, M, K, A, lda);
     K3_LAUNCHED();
     return K3HIP_OK;
 }
 
-template <int AM, bool F16, typename OUT>
+template <int AM>
 int launch(MidArgs &a, int M, int K, const void *A, long lda, hipStream_t st)
 {
     int ncu = 0, rc;
@@ -270,15 +258,14 @@ int launch(MidArgs &a, int M, int K, const void *A, long lda, hipStream_t st)
     long wide = 0;
     for (int i = 0; i < a.n; i++) wide += (a.s[i].rows + 127) / 128;
     // 128 x 128 once those tiles give every CU one: half the LDS reads per product. With two
-    // buffers, so that two workgroups share a CU (three: one). Hidden 4096, 16 x 64 heads, T =
-    // 1400: the layer 152 us, 174 on 64 x 128 tiles, 182 with three buffers; hidden 2048, 48 x 128,
-    // T = 300 the other way, 162 against 149 (294 tiles, 588).
+    // buffers, so that two workgroups share a CU (three: one). At K = 256: the table of the z
+    // product's rule in kda_layer.hip.
     if constexpr (AM == MID_A_16) {
-        if (wide * ((M + 127) / 128) >= ncu) return launch_tile<AM, 128, 128, 2, F16, OUT>(a, M, K, A, lda, st);
+        if (wide * ((M + 127) / 128) >= ncu) return launch_tile<AM, 128, 128, 2>(a, M, K, A, lda, st);
     }
     // 64 rows, and 128 columns once those tiles give every CU one; 64 below
-    if (wide * ((M + 63) / 64) >= ncu) return launch_tile<AM, 64, 128, 3, F16, OUT>(a, M, K, A, lda, st);
-    return launch_tile<AM, 64, 64, 5, F16, OUT>(a, M, K, A, lda, st);
+    if (wide * ((M + 63) / 64) >= ncu) return launch_tile<AM, 64, 128, 3>(a, M, K, A, lda, st);
+    return launch_tile<AM, 64, 64, 5>(a, M, K, A, lda, st);
 }
 
 }  // namespace
@@ -289,28 +276,22 @@ bool mid_supported(int K, const void *A, long lda, bool a_fp32)
            ((uintptr_t)A & 15) == 0;
 }
 
-int mid(int M, int K, int a_mode, const void *A, long lda, const MidSeg *segs, int n, bool f16, int out, hipStream_t st)
+int mid(int M, int K, int a_mode, const void *A, long lda, const MidSeg *segs, int n, hipStream_t st)
 {
     if (M <= 0 || n <= 0) return K3HIP_OK;
     if (n > MID_SEGS || !mid_supported(K, A, lda, a_mode != MID_A_16))
         K3_FAIL(K3HIP_EUNSUPPORTED, "mid: %d weights, K=%d (a multiple of %d), lda=%ld, or A misaligned", n, K, BK, lda);
-    if ((out != K3HIP_F32 && out != K3HIP_BF16) || (f16 && a_mode != MID_A_16))
-        K3_FAIL(K3HIP_EINVAL, "mid: output dtype %d, operands %d", out, a_mode);
     MidArgs a{};
-    const int es = out == K3HIP_F32 ? 4 : 2;
     for (int i = 0; i < n; i++) {
         MidSeg s = segs[i];
         if (s.rows <= 0) continue;
         if ((uintptr_t)s.B & 15) K3_FAIL(K3HIP_EUNSUPPORTED, "mid: weight %d misaligned", i);
         if (s.cols <= 0 || s.cols > s.rows) s.cols = s.rows;
-        s.vec = ((uintptr_t)s.C & (4 * es - 1)) == 0 && s.ldc % 4 == 0;
+        s.vec = ((uintptr_t)s.C & 15) == 0 && s.ldc % 4 == 0;
         a.s[a.n++] = s;
     }
     if (a.n == 0) return K3HIP_OK;
-    if (f16) return out == K3HIP_F32 ? launch<MID_A_16, true, float>(a, M, K, A, lda, st) : launch<MID_A_16, true, uint16_t>(a, M, K, A, lda, st);
-    if (out != K3HIP_F32) K3_FAIL(K3HIP_EINVAL, "mid: bf16 results on fp16 operands only");
-    if (a_mode == MID_A_16) return launch<MID_A_16, false, float>(a, M, K, A, lda, st);
-    return launch<MID_A_SPLIT, false, float>(a, M, K, A, lda, st);
+    return a_mode == MID_A_16 ? launch<MID_A_16>(a, M, K, A, lda, st) : launch<MID_A_SPLIT>(a, M, K, A, lda, st);
 }
 
 }  // namespace k3kda
