@@ -170,7 +170,7 @@ int gemm_rows_with_part(int B, int K, const float *x, long ldx, int N1, const ui
 // o [B][H VH] = (chat_h . W_UV_h^T) * sigmoid(g) with W_UV_h the rows
 // h (QN + VH) + QN .. + VH of kvb [H (QN + VH)][KL] (bf16) and g (may be nullptr) the gate
 // logits at row stride ldg; zout[0 .. zn) = 0 on the way (may be nullptr). Shapes:
-// mla_attention_supported (KL a multiple of 16 up to 512, CW a multiple of 4 up to
+// mla_attention_supported (H <= 64, KL a multiple of 16 up to 512, CW a multiple of 4 up to
 // 576), QN % 4 == 0, KL % 8 == 0, VH <= 128. ws: mla_attention_ws_bytes bytes, 256-byte aligned; A2, q,
 // cache and kvb 16-byte aligned.
 bool mla_attention_supported(int H, int KL, int CW);

@@ -23,7 +23,7 @@
 // attention the same way. The attention reads
 // the cache once where the shape fits the fused kernel (kda_mla_attn.hip: split-bf16 MFMA
 // scores, online softmax with the reference's scale (nope+rope)^-0.5, split-bf16 weighted
-// sum of the latents; kv_lora <= 512, kv_lora + rope <= 576); other shapes take
+// sum of the latents; heads <= 64, kv_lora <= 512, kv_lora + rope <= 576); other shapes take
 // two strided-batched fp32 GEMMs (scores, then P . cache) around the reference's softmax
 // (fp32 scores times (nope+rope)^-0.5, max, expf, double sum).
 #include <math.h>

@@ -10,10 +10,9 @@
 // kv_b absorbed. The cache (302 MB at 16 sequences x 8192 positions x 576 floats) dominates
 // the bytes, so the kernel reads it exactly once, and everything else stays on the chip:
 //
-//  * A workgroup (8 waves, two per SIMD) owns one sequence, up to 64 heads (more heads are
-//    dealt evenly over groups, which find the cache rows in L2 and the memory-side cache)
-//    and a contiguous range of positions (CUs / (B groups) ranges, rounded down so that one
-//    round of workgroups covers the GPU) and walks it in tiles of 16 positions (16
+//  * A workgroup (8 waves, two per SIMD) owns one sequence and a contiguous range of
+//    positions (CUs / B ranges per sequence, rounded down so that one round of workgroups
+//    covers the GPU) and walks it in tiles of 16 positions (16
 //    contiguous cache rows). Every thread loads its 16-byte units of a tile one iteration
 //    ahead into registers, splits them into bf16 hi/lo and stages them row-major in LDS
 //    (four tile buffers: the tile being scored, the two being summed, the next one).
@@ -82,9 +81,8 @@ constexpr size_t AT_P = (size_t)AT_NB * 2 * AT_PLANE * 2;  // bytes: tiles; then
 constexpr size_t AT_A = AT_P + 2 * 4 * 64 * 16;              // rescale factors [2][4][64] fp32
 constexpr size_t AT_LDS = AT_A + 2 * 4 * 64 * 4;
 
-// H heads in groups of HG (a multiple of 16, at most 64; the last may hold fewer)
 struct AtGeom {
-    int H, HG, CW, KL;
+    int H, CW, KL;
 };
 
 // Where the query rows come from: qcat[b][h] = [sum over planes p of A2[pB+b][h] (one plane from
@@ -102,19 +100,14 @@ __device__ __forceinline__ void split2(float a, float b, bf16x2 &hi, bf16x2 &lo)
     lo = __builtin_convertvector(f2{a - __uint_as_float(u << 16), b - __uint_as_float(u & 0xffff0000u)}, bf16x2);
 }
 
-// Workgroup (sp, b, z): positions [Tn sp / nsplit, Tn (sp + 1) / nsplit) of sequence b, heads
-// z HG .. of the group (h and H below count within it; h0 is its first). NHT: 16-head tiles
-// of a group, so that groups of fewer than 64 heads spend no products on absent ones (16 heads,
-// 16 sequences x 8192 positions, hidden 4096: the layer 118.7 -> 111.6 us). LL: the weighted sum
-// also takes the lo x lo products, for head counts beyond 64: two fp32 GEMMs around a softmax
-// served those before (96 heads, 3 sequences x 3001 positions: the layer 156.5 -> 127 us, 16
-// x 8192: 383 -> 219 us), and without them the layer's error against 64 bits was up to 15%
-// above theirs on short contexts.
+// Workgroup (sp, b): positions [Tn sp / nsplit, Tn (sp + 1) / nsplit) of sequence b. NHT: its
+// 16-head tiles, so that fewer than 64 heads spend no products on absent ones (16 heads, 16
+// sequences x 8192 positions, hidden 4096: the layer 118.7 -> 111.6 us).
 // Wave w: S role for w < 4 (head tile ht = w: heads 16 ht .. 16 ht + 15; lane l works for
 // head h = 16 ht + (l & 15), kg = l >> 4 picks its K slice in the score product and its 4
 // positions of each tile, 4 kg .. 4 kg + 3), U role otherwise (latent channel quarter
 // w - 4, all head tiles). FULL: kv_lora + rope = 576, every staging unit of a row exists.
-template <bool FULL, int NHT, bool LL>
+template <bool FULL, int NHT>
 __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void mla_attn_kernel(
     AtGeom g, int Tn, int cap, int nsplit, float scale2, AtQ qs,
     const float *__restrict__ cache, float *__restrict__ pctx, float *__restrict__ pm, float *__restrict__ pl)
@@ -127,8 +120,7 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     const int sp = blockIdx.x, b = blockIdx.y;
     const int p0 = (int)((long)Tn * sp / nsplit), p1 = (int)((long)Tn * (sp + 1) / nsplit);
     const int ntile = (p1 - p0 + AT_T - 1) / AT_T;
-    const int Hall = g.H, h0 = (int)blockIdx.z * g.HG, H = min(g.HG, Hall - h0);
-    const int CW = FULL ? 32 * AT_MAXKS : g.CW, KL = g.KL;
+    const int H = g.H, CW = FULL ? 32 * AT_MAXKS : g.CW, KL = g.KL;
     const int h = 16 * ht + m;
     const bool act = 16 * ht < H;   // wave-uniform: this wave has heads
 
@@ -184,7 +176,7 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
                 float x[8];
                 const int c = 32 * i + 8 * kg;
                 const bool ok = h < H;
-                const size_t bh = (size_t)b * Hall + h0 + (ok ? h : 0);
+                const size_t bh = (size_t)b * H + (ok ? h : 0);
                 const float *a2 = qs.A2 + bh * CW;
                 const float *qr = qs.q + bh * qs.QH + qs.QN - KL;
 #pragma unroll
@@ -195,7 +187,7 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
                         if (cc < KL) {
                             v = *reinterpret_cast<const f4 *>(a2 + cc);
                             for (int p = 1; p < qs.planes; p++)
-                                v += *reinterpret_cast<const f4 *>(a2 + (size_t)p * qs.B * Hall * CW + cc);
+                                v += *reinterpret_cast<const f4 *>(a2 + (size_t)p * qs.B * H * CW + cc);
                         } else v = *reinterpret_cast<const f4 *>(qr + cc);
                     }
                     x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
@@ -293,8 +285,8 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         lsum += __shfl_xor(lsum, 16, 64);
         lsum += __shfl_xor(lsum, 32, 64);
         if (act && h < H && kg == 0) {
-            pm[((size_t)b * nsplit + sp) * Hall + h0 + h] = M;
-            pl[((size_t)b * nsplit + sp) * Hall + h0 + h] = lsum;
+            pm[((size_t)b * nsplit + sp) * H + h] = M;
+            pl[((size_t)b * nsplit + sp) * H + h] = lsum;
         }
     } else {
         // U wave u = w - 4 owns latent channel tiles 8 u .. 8 u + 7 for all head tiles:
@@ -414,11 +406,6 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 #pragma unroll
                 for (int g2 = 0; g2 < NHT; g2++)
                     acc[jj][g2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, ph[g2], acc[jj][g2], 0, 0, 0);
-                if constexpr (LL) {
-#pragma unroll
-                    for (int g2 = 0; g2 < NHT; g2++)
-                        acc[jj][g2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, pq[g2], acc[jj][g2], 0, 0, 0);
-                }
 #pragma unroll
                 for (int g2 = 0; g2 < NHT; g2++)
                     acc[jj][g2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, pq[g2], acc[jj][g2], 0, 0, 0);
@@ -445,7 +432,7 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
             for (int g2 = 0; g2 < NHT; g2++) {
                 const int hh = 16 * g2 + m;
                 if (hh >= H) continue;
-                float *outp = pctx + (((size_t)b * nsplit + sp) * Hall + h0 + hh) * KL + 4 * kg;
+                float *outp = pctx + (((size_t)b * nsplit + sp) * H + hh) * KL + 4 * kg;
 #pragma unroll
                 for (int jj = 0; jj < AT_UCT; jj++) {
                     const int j = AT_UCT * u + jj;
@@ -592,36 +579,33 @@ int at_cus()
     return n;
 }
 
+// Up to 64 heads. More (two groups of heads over the same cache rows) ran here faster, 96 heads,
+// 3 sequences x 3001 positions: the layer 127 us against 155, but on 16 bits of the cache, the
+// query rows and the probabilities where the fp32 GEMMs of kda_mla.hip, which serve those shapes,
+// work on 24: with scores of spread 1 the layer was 5.7e-6 from 64 bits, 0.5e-6 on the GEMMs.
 bool at_geom(int H, int KL, int CW, AtGeom &g)
 {
-    if (H <= 0 || KL <= 0 || (KL % 16) || KL > 16 * AT_MAXCT || CW < KL || (CW % 4) ||
+    if (H <= 0 || H > 64 || KL <= 0 || (KL % 16) || KL > 16 * AT_MAXCT || CW < KL || (CW % 4) ||
         CW > 32 * AT_MAXKS)
         return false;
-    const int tiles = (H + 15) / 16, groups = (tiles + 3) / 4;
-    if (groups > 65535) return false;
     g.H = H;
-    g.HG = 16 * ((tiles + groups - 1) / groups);
     g.CW = CW;
     g.KL = KL;
     return true;
 }
 
 // One workgroup per CU at most: a count rounded up (24 sequences: 264 workgroups) runs a
-// second, nearly empty round. With several head groups, ranges a multiple of 8, so that the
-// groups of a range run on one XCD and share its L2's copy of the cache rows.
-int at_nsplit(int B, int H, int Tn)
+// second, nearly empty round.
+int at_nsplit(int B, int Tn)
 {
-    const int groups = ((H + 15) / 16 + 3) / 4;
-    int n = std::min({AT_MAXSPLIT, (int)std::max(1L, at_cus() / ((long)B * groups)), std::max(1, Tn / AT_T)});
-    if (groups > 1 && n > 8) n &= ~7;
-    return n;
+    return std::min({AT_MAXSPLIT, std::max(1, at_cus() / B), std::max(1, Tn / AT_T)});
 }
 
 }  // namespace
 
 size_t mla_attention_ws_bytes(int B, int H, int KL, int Tn)
 {
-    const int nsplit = at_nsplit(B, H, Tn);
+    const int nsplit = at_nsplit(B, Tn);
     const size_t r = (size_t)B * nsplit * H;
     return ((r * KL * 4 + 255) & ~(size_t)255) + 2 * ((r * 4 + 255) & ~(size_t)255);
 }
@@ -640,7 +624,7 @@ int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, co
     if (!at_geom(H, KL, CW, g))
         K3_FAIL(K3HIP_EUNSUPPORTED, "mla attention: heads=%d kv_lora=%d kv_lora+rope=%d outside the fused kernel", H, KL, CW);
     if (B <= 0 || Tn <= 0 || Tn > cap) K3_FAIL(K3HIP_EINVAL, "mla attention: B=%d Tn=%d cap=%d", B, Tn, cap);
-    const int nsplit = at_nsplit(B, H, Tn);
+    const int nsplit = at_nsplit(B, Tn);
     const size_t need = mla_attention_ws_bytes(B, H, KL, Tn);
     const int QH = QN + (CW - KL);
     if (!ws || ws_bytes < need || ((uintptr_t)ws & 255) || ((uintptr_t)cache & 15) || ((uintptr_t)A2 & 15) ||
@@ -652,17 +636,16 @@ int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, co
     float *pctx = (float *)ws;
     float *pm = (float *)((char *)ws + ((r * KL * 4 + 255) & ~(size_t)255));
     float *pl = (float *)((char *)pm + ((r * 4 + 255) & ~(size_t)255));
-    const int nht = g.HG / 16, groups = (H + g.HG - 1) / g.HG;
-    const void *kern;   // more than one group: three or four head tiles each
-#define K3_AT(F) (groups > 1 ? (nht == 3 ? (const void *)mla_attn_kernel<F, 3, true> : (const void *)mla_attn_kernel<F, 4, true>) \
-                  : nht == 1 ? (const void *)mla_attn_kernel<F, 1, false> : nht == 2 ? (const void *)mla_attn_kernel<F, 2, false> \
-                  : nht == 3 ? (const void *)mla_attn_kernel<F, 3, false> : (const void *)mla_attn_kernel<F, 4, false>)
+    const int nht = (H + 15) / 16;
+    const void *kern;
+#define K3_AT(F) (nht == 1 ? (const void *)mla_attn_kernel<F, 1> : nht == 2 ? (const void *)mla_attn_kernel<F, 2> \
+                  : nht == 3 ? (const void *)mla_attn_kernel<F, 3> : (const void *)mla_attn_kernel<F, 4>)
     kern = CW == 32 * AT_MAXKS ? K3_AT(true) : K3_AT(false);
 #undef K3_AT
     K3_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)AT_LDS));
     float scale2 = scale * AT_LOG2E;
     void *args[] = {&g, &Tn, &cap, (void *)&nsplit, &scale2, (void *)&qs, (void *)&cache, &pctx, &pm, &pl};
-    K3_HIP(hipLaunchKernel(kern, dim3(nsplit, B, groups), dim3(AT_NT), args, AT_LDS, st));
+    K3_HIP(hipLaunchKernel(kern, dim3(nsplit, B), dim3(AT_NT), args, AT_LDS, st));
     K3_LAUNCHED();
     hipLaunchKernelGGL(mla_attn_merge_kernel, dim3(H, B), dim3(128), 0, st, B, H, KL, nsplit, pctx, pm, pl, chat);
     K3_LAUNCHED();
