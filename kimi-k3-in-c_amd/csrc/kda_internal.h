@@ -3,6 +3,7 @@
 #pragma once
 
 #include "k3kda_common.h"
+#include "kda_scratch.h"
 
 namespace k3kda {
 
@@ -94,29 +95,7 @@ int decode_strided(int B, int H, int D, float *S, long s_stride, float *o, const
                    const float *k, const float *v, const float *alpha, const float *beta,
                    float qs, hipStream_t st);
 
-// Stream-ordered scratch of one call: a block kept between calls (kda_layer.hip) or
-// hipMallocAsync on `st`, given back in stream order when the StreamBuf goes.
-struct WsBlock {
-    void *p;
-    size_t size;
-    int dev;
-    hipStream_t last;   // stream of its last call
-    hipEvent_t ev;      // after that call; none for the null stream
-    bool busy;
-};
-void ws_return(WsBlock *k, hipStream_t st);
-// A weight set was uploaded (+1) or released (-1); blocks are kept only while any is there.
-void ws_handles(int d);
-struct StreamBuf {
-    void *p = nullptr;
-    hipStream_t st = nullptr;
-    WsBlock *kept = nullptr;
-    ~StreamBuf()
-    {
-        if (kept) ws_return(kept, st);
-        else if (p) (void)hipFreeAsync(p, st);
-    }
-};
+// scratch_alloc (kda_scratch.h) with the call's error set; refused inside a no-allocation entry point.
 int stream_alloc(StreamBuf &b, size_t bytes, hipStream_t st);
 
 // Decode copy of a row-major bf16 weight W[N][K] in MFMA fragment order, for gemm_rows:

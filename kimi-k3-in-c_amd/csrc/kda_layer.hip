@@ -17,7 +17,6 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
-#include <vector>
 
 #include "kda_internal.h"
 #include "kda_prep_math.h"
@@ -58,175 +57,14 @@ int zero_fill(float *p, size_t n, hipStream_t st)
 // call path would make is refused instead (the call then returns an error, allocating nothing).
 static thread_local bool g_no_alloc;
 
-// ------------------------------------------------------------------ workspaces ----
-// Scratch blocks kept between calls while any weight set is uploaded (handles > 0), since
-// hipMallocAsync + hipFreeAsync cost the host 10-11 us a pair, and after a synchronisation,
-// when the runtime's pool has given its memory back, 50 us for 64 MB and ~350 us for the 1.4 GB
-// of an 8192-token layer; a kept block costs ~1 us.
-//  * A block is handed to one call at a time (busy). Its next call is on the same stream, so
-//    stream order protects it, or the block is idle by its event.
-//  * The legacy null stream lives for ever, so equality of the handle is identity and no event
-//    is needed. Any other stream may be destroyed and its handle given to a new one: its blocks
-//    carry an event recorded after the call's last launch, waited for on reuse.
-//  * No call waits for another stream's block: it gets a new one while the device's blocks
-//    stay within WS_KEEP_BYTES (blocks too small for the call are given back first), and past
-//    that a plain stream allocation.
-//  * Calls being captured into a graph take plain stream allocations (the graph's own nodes).
-//  * The last release gives every block back, in stream order.
-constexpr size_t WS_KEEP_BYTES = 4ull << 30;   // per device, of 288 GB
-constexpr size_t WS_MIN_BLOCK = 1u << 20;
-
-namespace {
-
-struct WsPool {
-    std::mutex mu;
-    std::vector<WsBlock *> blocks;   // all of them, busy ones too
-    size_t held[64] = {};            // bytes per device
-    int handles = 0;
-};
-
-WsPool &ws_pool()
-{
-    static WsPool *p = new WsPool;   // never destroyed: calls may outlive static destructors
-    return *p;
-}
-
-// Sizes in steps of a quarter of a power of two, so that slowly growing requests share blocks.
-size_t ws_class(size_t bytes)
-{
-    if (bytes <= WS_MIN_BLOCK) return WS_MIN_BLOCK;
-    size_t step = WS_MIN_BLOCK / 4;
-    while (step * 8 < bytes) step *= 2;
-    return (bytes + step - 1) / step * step;
-}
-
-// Give block i back to the runtime in stream order; the pool is locked and the block not busy.
-void ws_drop(WsPool &P, size_t i)
-{
-    WsBlock *k = P.blocks[i];
-    int dev = 0;
-    const bool other = hipGetDevice(&dev) == hipSuccess && dev != k->dev && hipSetDevice(k->dev) == hipSuccess;
-    if (k->ev) {
-        (void)hipStreamWaitEvent(nullptr, k->ev, 0);
-        (void)hipEventDestroy(k->ev);
-    }
-    (void)hipFreeAsync(k->p, nullptr);
-    if (other) (void)hipSetDevice(dev);
-    P.held[k->dev] -= k->size;
-    delete k;
-    P.blocks.erase(P.blocks.begin() + (long)i);
-}
-
-// Event queries are kept out of the rules of a capture that another stream or thread may have
-// open in its global mode.
-struct RelaxedCapture {
-    hipStreamCaptureMode m = hipStreamCaptureModeRelaxed;
-    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&m); }
-    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&m); }
-};
-
-// A kept block of at least `bytes` for a call on st, or nullptr: take a plain allocation.
-WsBlock *ws_take(size_t bytes, hipStream_t st)
-{
-    WsPool &P = ws_pool();
-    int dev = 0;
-    if (st) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        hipDevice_t sd = 0;
-        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-            hipStreamGetDevice(st, &sd) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        dev = (int)sd;
-    } else if (hipGetDevice(&dev) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    const size_t size = ws_class(bytes);
-    if (dev < 0 || dev >= 64 || size > WS_KEEP_BYTES) return nullptr;
-    std::lock_guard<std::mutex> lock(P.mu);
-    if (P.handles <= 0) return nullptr;
-    RelaxedCapture relaxed;
-    WsBlock *best = nullptr;
-    for (WsBlock *k : P.blocks) {
-        if (k->busy || k->dev != dev || k->size < bytes || (best && best->size <= k->size)) continue;
-        if (k->last == st || (k->ev && hipEventQuery(k->ev) == hipSuccess)) best = k;
-    }
-    if (best && best->ev && hipStreamWaitEvent(st, best->ev, 0) != hipSuccess) best = nullptr;
-    (void)hipGetLastError();   // hipErrorNotReady of a query
-    if (!best) {
-        for (size_t i = P.blocks.size(); i-- > 0 && P.held[dev] + size > WS_KEEP_BYTES;)
-            if (P.blocks[i]->dev == dev && !P.blocks[i]->busy && P.blocks[i]->size < bytes) ws_drop(P, i);
-        if (P.held[dev] + size > WS_KEEP_BYTES) return nullptr;
-        void *p = nullptr;
-        if (hipMallocAsync(&p, size, st) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        best = new WsBlock{p, size, dev, st, nullptr, false};
-        P.blocks.push_back(best);
-        P.held[dev] += size;
-    }
-    best->busy = true;
-    best->last = st;
-    return best;
-}
-
-}  // namespace
-
-// After the call's last launch.
-void ws_return(WsBlock *k, hipStream_t st)
-{
-    WsPool &P = ws_pool();
-    std::lock_guard<std::mutex> lock(P.mu);
-    if (st) {
-        bool ok = k->ev || hipEventCreateWithFlags(&k->ev, hipEventDisableTiming) == hipSuccess;
-        if (ok) ok = hipEventRecord(k->ev, st) == hipSuccess;
-        if (!ok) {   // no event: wait here, once
-            (void)hipGetLastError();
-            (void)hipStreamSynchronize(st);
-        }
-    } else if (k->ev) {   // its next call is ordered by the null stream alone
-        (void)hipEventDestroy(k->ev);
-        k->ev = nullptr;
-    }
-    k->busy = false;
-    if (P.handles <= 0)
-        for (size_t i = 0; i < P.blocks.size(); i++)
-            if (P.blocks[i] == k) {
-                ws_drop(P, i);
-                break;
-            }
-}
-
-void ws_handles(int d)
-{
-    WsPool &P = ws_pool();
-    std::lock_guard<std::mutex> lock(P.mu);
-    P.handles += d;
-    if (P.handles <= 0)
-        for (size_t i = P.blocks.size(); i-- > 0;)
-            if (!P.blocks[i]->busy) ws_drop(P, i);
-}
-
 int stream_alloc(StreamBuf &b, size_t bytes, hipStream_t st)
 {
-    b.st = st;
     if (g_no_alloc)
         K3_FAIL(K3HIP_EINVAL, "no-allocation entry point: a step needs %zu bytes of scratch beyond the fixed "
                 "array", bytes);
     if (bytes == 0) bytes = 256;
-    if ((b.kept = ws_take(bytes, st))) {
-        b.p = b.kept->p;
-        return K3HIP_OK;
-    }
-    hipError_t e = hipMallocAsync(&b.p, bytes, st);
-    if (e != hipSuccess) {
-        b.p = nullptr;
-        (void)hipGetLastError();
-        K3_FAIL(K3HIP_ENOMEM, "hipMallocAsync(%zu bytes): %s", bytes, hipGetErrorString(e));
-    }
+    const hipError_t e = scratch_alloc(b, bytes, st);
+    if (e != hipSuccess) K3_FAIL(K3HIP_ENOMEM, "hipMallocAsync(%zu bytes): %s", bytes, hipGetErrorString(e));
     return K3HIP_OK;
 }
 
