@@ -229,7 +229,7 @@ extern "C" int k3hip_kda_upload_ex(const K3KdaW *w, const K3Cfg *c, int parts, k
     {
         void *blk = nullptr;
         const size_t need = dev_part_bytes(w, c);
-        if (hipMalloc(&blk, need) != hipSuccess) {
+        if (device_alloc(&blk, need) != hipSuccess) {
             (void)hipGetLastError();
             set_error("k3hip_kda_upload: hipMalloc(%zu bytes)", need);
             rc = K3HIP_ENOMEM;
@@ -246,7 +246,7 @@ extern "C" int k3hip_kda_upload_ex(const K3KdaW *w, const K3Cfg *c, int parts, k
     // [W | W] copies of f_b (P x 2D) and o (E x 2P) for the bf16 prefill path
     auto twice = [&](void **dst, const void *src, size_t rows, size_t cols) -> int {
         const size_t rb = cols * 2;
-        K3_HIP(hipMalloc(dst, rows * rb * 2));
+        K3_HIP(device_alloc(dst, rows * rb * 2));
         d->bytes += rows * rb * 2;
         K3_HIP(hipMemcpy2D(*dst, 2 * rb, src, rb, rb, rows, hipMemcpyDeviceToDevice));
         K3_HIP(hipMemcpy2D((char *)*dst + rb, 2 * rb, src, rb, rb, rows, hipMemcpyDeviceToDevice));
@@ -255,9 +255,9 @@ extern "C" int k3hip_kda_upload_ex(const K3KdaW *w, const K3Cfg *c, int parts, k
     // W_o as fp16 for the prefill o_proj (y is RMS-normalised, so fp16 holds it)
     auto to_f16 = [&](void **dst, const void *src, size_t n) -> int {
         int *bad = nullptr, hbad = 0;
-        K3_HIP(hipMalloc(dst, n * 2));
+        K3_HIP(device_alloc(dst, n * 2));
         d->bytes += n * 2;
-        K3_HIP(hipMalloc(&bad, sizeof(int)));
+        K3_HIP(device_alloc((void **)&bad, sizeof(int)));
         int r = K3HIP_OK;
         if (hipMemcpy(bad, &hbad, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) r = K3HIP_EHIP;
         if (r == K3HIP_OK) {
@@ -285,7 +285,7 @@ extern "C" int k3hip_kda_upload_ex(const K3KdaW *w, const K3Cfg *c, int parts, k
     }
     // fragment-ordered copies for the decode projections (row-major stays for prefill)
     auto frag = [&](void **dst, const void *src, int N, int Kd) -> int {
-        K3_HIP(hipMalloc(dst, rows_frag_elems(N, Kd) * 2));
+        K3_HIP(device_alloc(dst, rows_frag_elems(N, Kd) * 2));
         d->bytes += rows_frag_elems(N, Kd) * 2;
         return rows_frag_pack((const uint16_t *)src, N, Kd, (uint16_t *)*dst, nullptr);
     };

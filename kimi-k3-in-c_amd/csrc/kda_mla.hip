@@ -391,7 +391,7 @@ extern "C" int k3hip_mla_upload(const K3MlaW *w, const K3Cfg *c, k3hip_mla_weigh
     {
         const size_t rows[3] = {(size_t)d->QL, (size_t)(d->KL + d->QR), d->gate ? H * d->VH : 0};
         const void *src[3] = {w->q_a, w->kv_a, d->gate ? w->g : nullptr};
-        if (hipMalloc(&d->xin, N1 * E * 2) != hipSuccess) {
+        if (device_alloc(&d->xin, N1 * E * 2) != hipSuccess) {
             (void)hipGetLastError();
             d->xin = nullptr;
             k3hip_mla_release(d);
@@ -417,7 +417,7 @@ extern "C" int k3hip_mla_upload(const K3MlaW *w, const K3Cfg *c, k3hip_mla_weigh
     };
     for (auto &u : up) {
         if (!u.src) continue;
-        if (hipMalloc(u.dst, u.bytes) != hipSuccess || hipMemcpy(*u.dst, u.src, u.bytes, hipMemcpyHostToDevice) != hipSuccess) {
+        if (device_alloc(u.dst, u.bytes) != hipSuccess || hipMemcpy(*u.dst, u.src, u.bytes, hipMemcpyHostToDevice) != hipSuccess) {
             (void)hipGetLastError();
             k3hip_mla_release(d);
             K3_FAIL(K3HIP_ENOMEM, "k3hip_mla_upload: device copy of %zu bytes", u.bytes);
@@ -428,7 +428,7 @@ extern "C" int k3hip_mla_upload(const K3MlaW *w, const K3Cfg *c, k3hip_mla_weigh
     d->QNP = (d->QN + 31) / 32 * 32;
     if (d->QNP <= 256) {
         const size_t n = H * d->KL * d->QNP;
-        if (hipMalloc(&d->ukt, n * 2) != hipSuccess) {
+        if (device_alloc(&d->ukt, n * 2) != hipSuccess) {
             (void)hipGetLastError();
             d->ukt = nullptr;
             k3hip_mla_release(d);
@@ -447,7 +447,7 @@ extern "C" int k3hip_mla_upload(const K3MlaW *w, const K3Cfg *c, k3hip_mla_weigh
         {&d->xin, (int)N1, (int)E}, {&d->q_b, (int)(H * QH), d->QL}, {&d->o, (int)E, (int)(H * d->VH)}};
     for (auto &f : fr) {
         void *packed = nullptr;
-        if (hipMalloc(&packed, rows_frag_elems(f.N, f.K) * 2) != hipSuccess ||
+        if (device_alloc(&packed, rows_frag_elems(f.N, f.K) * 2) != hipSuccess ||
             rows_frag_pack((const uint16_t *)*f.w, f.N, f.K, (uint16_t *)packed, nullptr) != K3HIP_OK ||
             hipStreamSynchronize(nullptr) != hipSuccess) {
             (void)hipGetLastError();

@@ -27,5 +27,7 @@ struct StreamBuf {
 
 // b.p = at least `bytes` of device memory for work on st.
 hipError_t scratch_alloc(StreamBuf &b, size_t bytes, hipStream_t st);
+// hipMalloc for what outlives a call (weights, states).
+hipError_t device_alloc(void **p, size_t bytes);
 
 }  // namespace k3kda

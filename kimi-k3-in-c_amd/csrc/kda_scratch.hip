@@ -17,6 +17,8 @@
 //  * A block leaves the list only when the runtime has taken it back; where the wait for its last
 //    call or the free is refused it stays listed, counted and whole.
 //  * Calls being captured into a graph take plain stream allocations (the graph's own nodes).
+//  * Where an allocation fails, idle memory of the pool's must not be the reason: every block that
+//    no call holds goes back, the host waits for that, and the allocation is tried again.
 //  * The last release gives every block back: the null stream's on it, any other on a stream of
 //    this file's own behind its event, so no stream of the caller's waits. A block whose call is
 //    still being issued then goes back with that call.
@@ -135,20 +137,38 @@ hipStream_t ws_own_stream(WsPool &P, int dev)
     return P.own[dev];
 }
 
-// The last weight set has gone.
-void ws_give_all(WsPool &P)
+// Give back every block that no call holds, of one device or (-1) of all; blocks of the null
+// stream only with null_too, since that is work on it. The number given back.
+int ws_give_all(WsPool &P, int dev, bool null_too)
 {
     RelaxedCapture relaxed;
+    int n = 0;
     for (size_t i = P.blocks.size(); i-- > 0;) {
         const WsBlock *k = P.blocks[i];
-        if (k->busy) continue;
-        if (k->last == nullptr) {   // of the null stream: in its order, on its device
+        if (k->busy || (dev >= 0 && k->dev != dev)) continue;
+        if (k->last == nullptr) {   // in the null stream's order, on its device
             OnDevice d(k->dev);
-            if (d.good) (void)ws_give(P, i, nullptr);
+            n += null_too && d.good && ws_give(P, i, nullptr);
         } else if (hipStream_t own = ws_own_stream(P, k->dev)) {
-            (void)ws_give(P, i, own);
+            n += ws_give(P, i, own);
         }
     }
+    return n;
+}
+
+// The device's memory that no call holds, back with the device for an allocation for st that has
+// failed. False: there was none.
+bool ws_trim(int dev, hipStream_t st)
+{
+    WsPool &P = ws_pool();
+    std::lock_guard<std::mutex> lock(P.mu);
+    if (ws_give_all(P, dev, st == nullptr) == 0) return false;
+    OnDevice d(dev);
+    if (P.own[dev]) (void)ok(hipStreamSynchronize(P.own[dev]));
+    if (!st) (void)ok(hipStreamSynchronize(nullptr));
+    hipMemPool_t pool = nullptr;   // the runtime keeps freed memory until it is trimmed
+    if (ok(hipDeviceGetDefaultMemPool(&pool, dev))) (void)ok(hipMemPoolTrimTo(pool, 0));
+    return true;
 }
 
 // The device of st; false while st is being captured or where it cannot be told.
@@ -232,7 +252,7 @@ void ws_handles(int d)
     WsPool &P = ws_pool();
     std::lock_guard<std::mutex> lock(P.mu);
     P.handles += d;
-    if (P.handles <= 0) ws_give_all(P);
+    if (P.handles <= 0) (void)ws_give_all(P, -1, true);
 }
 
 hipError_t scratch_alloc(StreamBuf &b, size_t bytes, hipStream_t st)
@@ -242,11 +262,27 @@ hipError_t scratch_alloc(StreamBuf &b, size_t bytes, hipStream_t st)
         b.p = b.kept->p;
         return hipSuccess;
     }
-    const hipError_t e = hipMallocAsync(&b.p, bytes, st);
+    hipError_t e = hipMallocAsync(&b.p, bytes, st);
     if (e != hipSuccess) {
-        b.p = nullptr;
         (void)hipGetLastError();
+        int dev = 0;
+        if (ws_device(st, dev) && ws_trim(dev, st) && (e = hipMallocAsync(&b.p, bytes, st)) != hipSuccess)
+            (void)hipGetLastError();
     }
+    if (e != hipSuccess) b.p = nullptr;
+    return e;
+}
+
+hipError_t device_alloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        int dev = 0;
+        if (ws_device(nullptr, dev) && ws_trim(dev, nullptr) && (e = hipMalloc(p, bytes)) != hipSuccess)
+            (void)hipGetLastError();
+    }
+    if (e != hipSuccess) *p = nullptr;
     return e;
 }
 

@@ -45,7 +45,7 @@ extern "C" int k3hip_kda_states_create(const K3Cfg *c, int n_layers, k3hip_kda_s
     s->layers = n_layers;
     s->kper = kper;
     const size_t bytes = kper * (size_t)n_layers * sizeof(float);
-    if (hipMalloc((void **)&s->d, bytes) != hipSuccess) {
+    if (device_alloc((void **)&s->d, bytes) != hipSuccess) {
         (void)hipGetLastError();
         free(s);
         K3_FAIL(K3HIP_ENOMEM, "k3hip_kda_states_create: hipMalloc(%zu bytes)", bytes);

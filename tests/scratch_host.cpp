@@ -29,8 +29,14 @@ struct Alloc {
 
 static Stream g_null;
 static std::map<void *, Alloc> g_live;
+struct Freed {
+    Stream *s;
+    size_t bytes;
+    bool synced;
+};
+static std::vector<Freed> g_freed;          // with the runtime's pool until it is trimmed after a wait
 static size_t g_bytes, g_limit = ~(size_t)0;
-static int g_violations, g_null_in_capture, g_waits, g_refuse_wait, g_refuse_free, g_refuse_record, g_refuse_sync, g_trims;
+static int g_violations, g_null_in_capture, g_waits, g_refuse_wait, g_refuse_free, g_refuse_record, g_refuse_sync;
 static std::vector<Stream *> g_streams;
 static bool g_relaxed;
 
@@ -76,7 +82,9 @@ extern "C" {
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t st)
 {
     null_work(S(st));
-    if (g_bytes + n > g_limit) return hipErrorOutOfMemory;
+    size_t kept = 0;
+    for (auto &f : g_freed) kept += f.bytes;
+    if (g_bytes + kept + n > g_limit) return hipErrorOutOfMemory;
     *p = std::malloc(1);
     g_live[*p] = Alloc{n, {}};
     g_bytes += n;
@@ -89,6 +97,7 @@ hipError_t hipFreeAsync(void *p, hipStream_t st)
     null_work(S(st));
     if (!ordered(p, S(st))) g_violations++;
     g_bytes -= g_live.at(p).bytes;
+    g_freed.push_back({S(st), g_live.at(p).bytes, false});
     g_live.erase(p);
     return hipSuccess;
 }
@@ -140,6 +149,7 @@ hipError_t hipStreamSynchronize(hipStream_t st)
     for (auto &a : s->after)
         if (a.first->done < a.second) a.first->done = a.second;
     finish(s);
+    for (auto &f : g_freed) f.synced |= f.s == s;
     return hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *st, unsigned f) { return *st = H(make(f != hipStreamNonBlocking)), hipSuccess; }
@@ -151,7 +161,14 @@ hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *m)
     return hipSuccess;
 }
 hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t *p, int) { return *p = nullptr, hipSuccess; }
-hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { return g_trims++, hipSuccess; }
+hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t)
+{
+    std::vector<Freed> left;
+    for (auto &f : g_freed)
+        if (!f.synced) left.push_back(f);
+    g_freed.swap(left);
+    return hipSuccess;
+}
 }
 
 static int g_failed;
@@ -286,6 +303,45 @@ static void capture()
     a->capturing = false;
 }
 
+static void out_of_memory()
+{
+    Stream *a = make(false), *b = make(false), *c = make(false);
+    hipError_t e;
+    g_limit = 1000 * MB;
+    call(a, 256 * MB);                // held, in flight
+    call(&g_null, 256 * MB);          // the null stream's: not touched from another
+    void *held = nullptr;
+    {
+        StreamBuf busy;
+        CHECK(scratch_alloc(busy, 128 * MB, H(c)) == hipSuccess);
+        launch(c, held = busy.p);
+        call(b, 600 * MB, &e);        // fits without the idle 256
+        CHECK(e == hipSuccess && g_live.count(held));
+        call(b, 900 * MB, &e);        // does not fit
+        CHECK(e == hipErrorOutOfMemory && g_live.count(held));
+    }
+    (void)hipStreamSynchronize(H(b)); // the 600 MB of b's plain call
+    call(&g_null, 1000 * MB, &e);     // without everything idle, the null stream's own too
+    CHECK(e == hipSuccess);
+    g_limit = 2000 * MB;
+    call(a, 512 * MB);
+    void *w = nullptr;
+    CHECK(device_alloc(&w, 1900 * MB) == hipSuccess);   // weights
+    CHECK(device_alloc(&w, 1900 * MB) == hipErrorOutOfMemory && !w);
+}
+
+static void out_of_memory_under_capture()
+{
+    Stream *a = make(false), *b = make(false);
+    hipError_t e;
+    g_limit = 1000 * MB;
+    call(a, 512 * MB);
+    b->capturing = true;
+    call(b, 600 * MB, &e);            // the graph's allocation: nothing is waited for
+    CHECK(e == hipErrorOutOfMemory && a->done < a->issued);
+    b->capturing = false;
+}
+
 int main(int argc, char **argv)
 {
     struct { const char *name; void (*run)(); } tests[] = {
@@ -293,7 +349,7 @@ int main(int argc, char **argv)
         {"evict_idle_blocks_on_the_calls_stream", evict_idle_blocks_on_the_calls_stream},
         {"evict_own_block_in_flight", evict_own_block_in_flight}, {"refused_wait", refused_wait},
         {"refused_free", refused_free}, {"refused_record", refused_record}, {"last_release", last_release},
-        {"capture", capture},
+        {"capture", capture}, {"out_of_memory", out_of_memory}, {"out_of_memory_under_capture", out_of_memory_under_capture},
     };
     if (argc < 2) {
         for (auto &t : tests) std::printf("%s\n", t.name);
