@@ -9,7 +9,7 @@
 //   bf16 rows (the z product of the bf16 prefill, on f_a's split rows),
 //   fp32 rows split into bf16 hi + lo, both against the bf16 weight (fp32 accuracy: x = hi + lo
 //   to 2.5e-6 relative rms), which needs no split rows or second half of the result in memory
-//   (the full-accuracy layer).
+//   (the full-accuracy layer; the bits of kda_mm.hip on split rows and the two halves' sum).
 //
 // The 256 x 256 tiles of kda_mm.hip leave most of the GPU idle here (333 tokens of a hidden
 // 2048, 16 x 128 layer: 2 x 33 tiles over 256 CUs, and 16 for z), and a launch per weight
@@ -154,11 +154,15 @@ __global__ __launch_bounds__(NT, 2) void mid_kernel(const MidArgs ar, int M, int
 
     const int r16 = lane & 15, kq = lane >> 4;
     const int fo[2] = {r16 * ROW + ((kq ^ swz(r16)) << 4), r16 * ROW + (((4 + kq) ^ swz(r16)) << 4)};
-    f32x4 acc[TI][TJ];
+    // the lo halves' products have an accumulator of their own: added to the hi halves' once, at
+    // the end, they are not rounded to its last place at every step
+    f32x4 acc[PARTS][TI][TJ];
 #pragma unroll
-    for (int i = 0; i < TI; i++)
+    for (int p = 0; p < PARTS; p++)
 #pragma unroll
-        for (int j = 0; j < TJ; j++) acc[i][j] = 0.0f;
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) acc[p][i][j] = 0.0f;
 
     if constexpr (AM != MID_A_16) load_a32(0);
 #pragma unroll
@@ -201,7 +205,7 @@ __global__ __launch_bounds__(NT, 2) void mid_kernel(const MidArgs ar, int M, int
 #pragma unroll
                 for (int i = 0; i < TI; i++)
 #pragma unroll
-                    for (int j = 0; j < TJ; j++) acc[i][j] = mfma(b[s][j], a[s][p][i], acc[i][j]);
+                    for (int j = 0; j < TJ; j++) acc[p][i][j] = mfma(b[s][j], a[s][p][i], acc[p][i][j]);
         if constexpr (AM != MID_A_16) put_a32(ks + 1);
     }
     wait_vm<0>();   // no load may still be writing this workgroup's LDS when it ends
@@ -215,7 +219,8 @@ __global__ __launch_bounds__(NT, 2) void mid_kernel(const MidArgs ar, int M, int
 #pragma unroll
         for (int j = 0; j < TJ; j++) {
             const int n = n0 + wn * (BN / 2) + 16 * j + 4 * kq;
-            const f32x4 v = acc[i][j];
+            f32x4 v = acc[0][i][j];
+            if constexpr (PARTS == 2) v += acc[1][i][j];
             if (sg.vec && n + 4 <= sg.cols) {
                 *reinterpret_cast<f32x4 *>(sg.C + (long)m * sg.ldc + n) = v;
                 continue;

@@ -97,3 +97,27 @@ def test_short_prefill_projections_vs_oracle(gpu, hidden, H, D, Ts, dev):
             assert_close(got[P * D:], st_ref[P * D:], 1e-5 * rms(st_ref[P * D:]), 1e-5, f"T={T} conv history")
         print(f"hidden={hidden} H={H} D={D} T={T} {'dev' if dev else 'prefill'}: worst {r:.3f}x", flush=True)
     dw.close()
+
+
+def test_split_rows_and_tiles_give_the_same_bits(gpu):
+    """The full-accuracy layer's longest prefills (from 4e11 products of the input projections) run
+    kda_mm.hip on 2T split rows and add the halves, shorter ones kda_mid.hip with an accumulator
+    per half: a sequence in one call of the first kind and in two of the second (chunk boundaries do
+    not move) is the same bits."""
+    import torch
+    hidden, H, D, K, T = 4096, 32, 128, 4, 6016
+    P = H * D
+    assert T / 2 * (4 * P + D + H) * hidden < 4e11 < T * (4 * P + D + H) * hidden and T // 2 % 64 == 0
+    cfg = ko.make_cfg(hidden, H, D, K, -5.0, 1e-5)
+    dw = gpu.DeviceWeights(layer_weights(np.random.default_rng(9), hidden, H, D, K).w, cfg, gpu.UPLOAD_DEV)
+    x = torch.randn((T, hidden), device="cuda", generator=torch.Generator(device="cuda").manual_seed(9))
+    got = []
+    for n in (T, T // 2):
+        st, out = torch.zeros(P * D + 3 * P * (K - 1), device="cuda"), torch.empty_like(x)
+        for t in range(0, T, n):
+            dw.layer(out[t:t + n], x[t:t + n], st, n)
+        torch.cuda.synchronize()
+        assert torch.isfinite(out).all()
+        got.append((out, st))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    dw.close()
