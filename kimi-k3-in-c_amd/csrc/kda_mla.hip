@@ -104,7 +104,7 @@ struct LatRow {
 // The absorb product A2[r][h][c] = sum_k x[r][h QH + k] W_UK_h[k][c] for the M = B rows of x
 // (q, fp32, row stride ldx), split into bf16 hi + mid + lo (all 24 bits) as they are read, and
 // every head h: one 16 x 16 x 32 bf16 MFMA tile chain per wave (16 latent columns of
-// one head, the M rows in tiles of 16, lo to hi, K-steps of 32 in order), fp32 results at
+// one head, the M rows in tiles of 16, hi apart from mid and lo, K-steps of 32 in order), fp32 results at
 // A2 + r ldc + h CW + c. (Split rows written by the q_b product cost it three scattered 2-byte
 // stores an element and this kernel a third more loads.) Workgroup (x, h) takes
 // columns 64 x .. 64 x + 63 of head h. VEC: x's rows and head offsets are 16-byte aligned
@@ -176,11 +176,15 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, 
         mla_bf16x8 af[3][KS];
 #pragma unroll
         for (int t = 0; t < KS; t++) bsplit::split_row8(xa[t], xb[t], af[0][t], af[1][t], af[2][t]);
-        mla_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+        // the hi parts' products in an accumulator of their own, the small ones added at the end
+        mla_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f}, rest = c;
 #pragma unroll
-        for (int p = 2; p >= 0; p--)
+        for (int t = 0; t < KS; t++) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][t], bf[t], c, 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < KS; t++) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], bf[t], c, 0, 0, 0);
+        for (int p = 2; p >= 1; p--)
+#pragma unroll
+            for (int t = 0; t < KS; t++) rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], bf[t], rest, 0, 0, 0);
+        c += rest;
         // C layout: lane l holds rows 4 (l / 16) + i of the tile, column l % 16
 #pragma unroll
         for (int i = 0; i < 4; i++) {
