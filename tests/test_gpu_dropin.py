@@ -134,12 +134,14 @@ def test_dropin_int8_weights_vs_oracle(gpu, hidden, H, D, K, Ts):
     dw.close()
 
 
-@pytest.mark.parametrize("hidden,H,D,K,Ts", [(256, 2, 128, 4, (40, 1, 300)), (512, 4, 64, 3, (17, 64))])
+@pytest.mark.parametrize("hidden,H,D,K,Ts", [(256, 2, 128, 4, (40, 1, 300)), (512, 4, 64, 3, (17, 64)),
+                                             (512, 4, 64, 3, (33, 32, 64))])
 def test_dropin_bf16_prefill_mfma_vs_oracle(gpu, hidden, H, D, K, Ts):
-    """bf16 weights on prefills of T >= 16 take the MFMA projections (x split into bf16 hi + lo,
-    the two fp32 products added); the layer stays at the reference's decode bar (rtol 1e-4,
-    atol 1e-4 * rms) against the oracle's k3_kda_layer, on the host drop-in and on
-    k3hip_kda_layer_dev, with the state carried through a T = 1 call in between."""
+    """bf16 weights on prefills of T >= 33 take the MFMA projections (x split into bf16 hi + lo,
+    the two fp32 products added), shorter ones the double products (17 and 32 tokens here); the
+    layer stays at the reference's decode bar (rtol 1e-4, atol 1e-4 * rms) against the oracle's
+    k3_kda_layer, on the host drop-in and on k3hip_kda_layer_dev, with the state carried through a
+    T = 1 call in between."""
     import torch
     from test_gpu_layer_prefill import layer_weights
     rng = np.random.default_rng(0x4B334441 + 16 + hidden + D)

@@ -2,12 +2,14 @@
 """The double-accumulating projections of k3hip_kda_layer_dev (csrc/kda_proj.hip) at the edges
 of their forms: token counts around the GEMV / MFMA switch (4 | 5) and the 16-token tiles,
 hidden widths below, at and past one 512-wide block with and without whole 8-element slices,
-row counts on both sides of the one / two rows a wave rule (8192), each weight format.
+row counts on both sides of the one / two rows a wave rule (8192), two rows a wave over one block,
+over five and over seven (four at a time, then two, then the last with one slice), each weight
+format.
 
 The layer's conv history holds the last K - 1 projected q, k, v: double sums rounded once to
 fp32 (int8: the double sum of the int8 products rounded to fp32, times the row's fp32 scale).
 They are compared with the same sums by numpy in float64, whose other order moves the double
-sum by far less than 1e-9 for at most 1104 products of order one: at most one unit in the last
+sum by far less than 1e-9 for at most 3080 products of order one: at most one unit in the last
 place, 2^-23 relative (two for int8, whose product with the scale rounds once more). Output and
 state are held to the oracle's k3_kda_layer at the layer's 1e-4 bar.
 """
@@ -38,7 +40,8 @@ def project(w, wdt, hidden, x):
 @pytest.mark.parametrize("wdt", ["fp32", "bf16", "int8"])
 @pytest.mark.parametrize("hidden,H,D,Ts", [(72, 3, 64, (1, 2, 3, 4, 5, 16, 17, 32, 33, 70)),
                                            (100, 2, 64, (1, 3, 5, 20)), (1104, 1, 128, (4, 1, 15, 49, 65)),
-                                           (136, 16, 128, (1, 2, 4))])
+                                           (136, 16, 128, (1, 2, 4)), (2056, 16, 128, (1, 2, 3)),
+                                           (3080, 16, 128, (1, 2, 4))])
 def test_projection_forms_vs_oracle(gpu, hidden, H, D, Ts, wdt):
     import torch
     rng = np.random.default_rng(0x4B334441 + 0x90 + hidden + D)

@@ -45,6 +45,13 @@ def test_workspaces_of_calls_in_flight(gpu, threads):
         want.append((o, states[i].clone()))
 
     def rounds(k):
+        try:
+            compared.append(_rounds(k))
+        except BaseException as e:          # an exception would end in the thread: it fails the test here
+            bad.append((k, repr(e)))
+
+    def _rounds(k):
+        done = 0
         own = [torch.empty(n, device="cuda") for _ in lens]
         for r in range(3):
             streams = [torch.cuda.Stream(), torch.cuda.Stream()] + ([] if k else [cur])
@@ -54,8 +61,11 @@ def test_workspaces_of_calls_in_flight(gpu, threads):
             for i in range(len(lens)):
                 if not (torch.equal(outs[i], want[i][0]) and torch.equal(own[i], want[i][1])):
                     bad.append((k, r, i))
+                done += 1
+        return done
 
     bad: list = []
+    compared: list = []
     torch.cuda.synchronize()
     if threads:
         ts = [threading.Thread(target=rounds, args=(k + 1,)) for k in range(threads)]
@@ -67,3 +77,4 @@ def test_workspaces_of_calls_in_flight(gpu, threads):
         rounds(0)
     dw.close()
     assert not bad, bad
+    assert compared == [3 * len(lens)] * max(threads, 1)
