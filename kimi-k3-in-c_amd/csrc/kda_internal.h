@@ -141,8 +141,8 @@ int gemm_rows_with_part(int B, int K, const float *x, long ldx, int N1, const ui
                         size_t ws_floats = 0);
 
 // Attention of an absorbed MLA decode step (kda_mla_attn.hip) in one pass over the cache:
-// the query rows qcat[b][h] = [sum over `planes` p of A2[pB+b][h] | q_rope(b, h)] are formed in
-// the kernel from the absorb product A2 [planes B][H CW] (first KL of each head's CW columns) and
+// the query rows qcat[b][h] = [A2[b][h] | q_rope(b, h)] are formed in the kernel from the absorb
+// product A2 [B][H CW] (first KL of each head's CW columns) and
 // q [B][H][QN + CW - KL] (rope at column QN); cache [B][cap][CW] fp32 (latent = channels
 // 0..KL-1), positions 0..Tn-1; chat = softmax(scale qcat . cache^T) . latent (its position
 // ranges merged into chat [B][H KL], 16-byte aligned), then
@@ -154,7 +154,7 @@ int gemm_rows_with_part(int B, int K, const float *x, long ldx, int N1, const ui
 // cache and kvb 16-byte aligned.
 bool mla_attention_supported(int H, int KL, int CW);
 size_t mla_attention_ws_bytes(int B, int H, int KL, int Tn);
-int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, int planes, const float *q,
+int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, const float *q,
                   int QN, const float *cache, const uint16_t *kvb, int VH, const float *g, long ldg, float *o, float *zout, size_t zn,
                   float *chat, void *ws, size_t ws_bytes, hipStream_t st);
 

@@ -40,12 +40,12 @@ struct k3hip_mla_weights {
     // q_a, kv_a and g (when gated) are row blocks of one matrix xin ([QL + KL + QR + H*VH]
     // [hidden], in that order): one pass over them projects a decode step's input. xin, q_b
     // and o are stored in MFMA fragment order for the few-rows GEMM (kda_rows.hip); kv_b
-    // stays row-major (bf16) for the head-batched absorb GEMMs.
+    // stays row-major (bf16) for the W_UV product.
     void *xin, *q_b, *kv_b, *o;
     float *q_a_norm, *kv_a_norm;
     // W_UK_h^T per head, [H][KL][QNP] bf16 with QNP = QN rounded up to 32 (zeros past QN): the
     // B operand of the absorb product, each lane's 8 consecutive K values one 16-byte load
-    void *ukt;   // nullptr when qk_nope > 256
+    void *ukt;
     int QNP;
 };
 
@@ -110,15 +110,17 @@ struct LatRow {
 // columns 64 x .. 64 x + 63 of head h. VEC: x's rows and head offsets are 16-byte aligned
 // and QN is a multiple of 8 (QH and ldx multiples of 4), so each lane's 8 K values are
 // one load or none. Workgroups (x, y) with y >= H write one latent row each.
-// KS = QNP / 32 K-steps, a template constant so that a tile's loads are
+// KS K-steps, a template constant so that a tile's loads are
 // issued together and waited for once (with a run-time count each load waited alone: 5.9 us).
+// QN up to 256: KS = QNP / 32, W_UK's fragments kept over the tiles of rows. Wider heads (WIDE) take
+// QNP in nk equal parts of 32 KS, whose registers are reused; the sums go on in the same order.
 typedef __bf16 mla_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mla_f32x4 __attribute__((ext_vector_type(4)));
-template <bool VEC, int KS>
+template <bool VEC, int KS, bool WIDE>
 __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, int KL, int CW,
                                                          const float *__restrict__ x, long ldx,
                                                          const uint16_t *__restrict__ ukt, float *__restrict__ A2,
-                                                         long ldc, int H, LatRow lr)
+                                                         long ldc, int H, int nk, LatRow lr)
 {
     if ((int)blockIdx.y >= H) {
         __shared__ double red[16];
@@ -139,51 +141,58 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, 
         }
         return;
     }
-    constexpr int QNP = 32 * KS;
+    const int QNP = 32 * KS * (WIDE ? nk : 1);
     const int h = blockIdx.y, lane = threadIdx.x & 63;
     const int n0 = 64 * blockIdx.x + 16 * (threadIdx.x >> 6);
-    if (n0 >= KL) return;   // wave-uniform; no barrier in this kernel
+    if (n0 >= KL) return;   // wave-uniform; no barrier from here on
     const int col = n0 + (lane & 15), kq = 8 * (lane >> 4);
     const bool cok = col < KL;
     const uint16_t *brow = ukt + ((size_t)h * KL + (cok ? col : 0)) * QNP + kq;
     mla_bf16x8 bf[KS];
+    auto load_b = [&](int k0) {
 #pragma unroll
-    for (int t = 0; t < KS; t++) bf[t] = *reinterpret_cast<const mla_bf16x8 *>(brow + 32 * t);
+        for (int t = 0; t < KS; t++) bf[t] = *reinterpret_cast<const mla_bf16x8 *>(brow + k0 + 32 * t);
+    };
+    if constexpr (!WIDE) load_b(0);
     for (int m0 = 0; m0 < M; m0 += 16) {
         const int r = m0 + (lane & 15);
         const float *xr = x + (size_t)(r < M ? r : 0) * ldx + (size_t)h * QH + kq;
-        f4 xa[KS], xb[KS];
-#pragma unroll
-        for (int t = 0; t < KS; t++) {
-            if constexpr (VEC) {
-                // QN % 8 == 0: an 8-value group is wholly inside or past QN; a group past it (or
-                // a row past M) loads the head's first group instead and is zeroed, so every
-                // load is issued unconditionally from an address inside the row
-                const bool ok = r < M && 32 * t + kq < QN;
-                const f4 *p = reinterpret_cast<const f4 *>(xr + (ok ? 32 * t : -kq));
-                xa[t] = p[0];
-                xb[t] = p[1];
-                if (!ok) xa[t] = xb[t] = f4(0.0f);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const float v = r < M && 32 * t + kq + e < QN ? xr[32 * t + e] : 0.0f;
-                    if (e < 4) xa[t][e] = v;
-                    else xb[t][e - 4] = v;
-                }
-            }
-        }
-        mla_bf16x8 af[3][KS];
-#pragma unroll
-        for (int t = 0; t < KS; t++) bsplit::split_row8(xa[t], xb[t], af[0][t], af[1][t], af[2][t]);
         // the hi parts' products in an accumulator of their own, the small ones added at the end
         mla_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f}, rest = c;
+        for (int k0 = 0; k0 < QNP; k0 += 32 * KS) {
+            if constexpr (WIDE) load_b(k0);
+            f4 xa[KS], xb[KS];
 #pragma unroll
-        for (int t = 0; t < KS; t++) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][t], bf[t], c, 0, 0, 0);
+            for (int t = 0; t < KS; t++) {
+                const int k = k0 + 32 * t;
+                if constexpr (VEC) {
+                    // QN % 8 == 0: an 8-value group is wholly inside or past QN; a group past it (or
+                    // a row past M) loads the head's first group instead and is zeroed, so every
+                    // load is issued unconditionally from an address inside the row
+                    const bool ok = r < M && k + kq < QN;
+                    const f4 *p = reinterpret_cast<const f4 *>(xr + (ok ? k : -kq));
+                    xa[t] = p[0];
+                    xb[t] = p[1];
+                    if (!ok) xa[t] = xb[t] = f4(0.0f);
+                } else {
 #pragma unroll
-        for (int p = 2; p >= 1; p--)
+                    for (int e = 0; e < 8; e++) {
+                        const float v = r < M && k + kq + e < QN ? xr[k + e] : 0.0f;
+                        if (e < 4) xa[t][e] = v;
+                        else xb[t][e - 4] = v;
+                    }
+                }
+            }
+            mla_bf16x8 af[3][KS];
 #pragma unroll
-            for (int t = 0; t < KS; t++) rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], bf[t], rest, 0, 0, 0);
+            for (int t = 0; t < KS; t++) bsplit::split_row8(xa[t], xb[t], af[0][t], af[1][t], af[2][t]);
+#pragma unroll
+            for (int t = 0; t < KS; t++) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][t], bf[t], c, 0, 0, 0);
+#pragma unroll
+            for (int p = 2; p >= 1; p--)
+#pragma unroll
+                for (int t = 0; t < KS; t++) rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][t], bf[t], rest, 0, 0, 0);
+        }
         c += rest;
         // C layout: lane l holds rows 4 (l / 16) + i of the tile, column l % 16
 #pragma unroll
@@ -194,23 +203,37 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(int M, int QH, int QN, 
     }
 }
 
+// Parts of at most eight 32-wide K-steps that a head's QN values are taken in, and the padded
+// length of a row of ukt: equal parts of whole steps.
+static int absorb_parts(int QN) { return (QN + 255) / 256; }
+static int absorb_row(int QN)
+{
+    const int nk = absorb_parts(QN), steps = (QN + 31) / 32;
+    return 32 * nk * ((steps + nk - 1) / nk);
+}
+
 template <bool VEC>
 static int mla_absorb_v(int M, int H, int QH, int QN, int QNP, int KL, int CW, const float *x, long ldx,
                         const uint16_t *ukt, float *A2, long ldc, const LatRow &lr, hipStream_t st)
 {
     const int gx = (KL + 63) / 64;
     const dim3 grid((unsigned)gx, (unsigned)(H + (lr.src ? (lr.B + gx - 1) / gx : 0)));
-#define K3_ABS(KS) hipLaunchKernelGGL((mla_absorb_kernel<VEC, KS>), grid, dim3(256), 0, st, M, QH, QN, KL, CW, x, ldx, ukt, A2, ldc, H, lr)
-    switch (QNP / 32) {
-    case 1: K3_ABS(1); break;
-    case 2: K3_ABS(2); break;
-    case 3: K3_ABS(3); break;
-    case 4: K3_ABS(4); break;
-    case 5: K3_ABS(5); break;
-    case 6: K3_ABS(6); break;
-    case 7: K3_ABS(7); break;
-    case 8: K3_ABS(8); break;
-    default: K3_FAIL(K3HIP_EUNSUPPORTED, "mla absorb: qk_nope padded to %d above 256", QNP);
+#define K3_ABS(KS, WIDE) hipLaunchKernelGGL((mla_absorb_kernel<VEC, KS, WIDE>), grid, dim3(256), 0, st, M, QH, QN, KL, CW, x, ldx, ukt, A2, ldc, H, nk, lr)
+    const int nk = absorb_parts(QN);   // nk > 1: more than 256 values, more than four steps a part
+    switch (QNP / 32 / nk + (nk > 1 ? 8 : 0)) {
+    case 1: K3_ABS(1, false); break;
+    case 2: K3_ABS(2, false); break;
+    case 3: K3_ABS(3, false); break;
+    case 4: K3_ABS(4, false); break;
+    case 5: K3_ABS(5, false); break;
+    case 6: K3_ABS(6, false); break;
+    case 7: K3_ABS(7, false); break;
+    case 8: K3_ABS(8, false); break;
+    case 13: K3_ABS(5, true); break;
+    case 14: K3_ABS(6, true); break;
+    case 15: K3_ABS(7, true); break;
+    case 16: K3_ABS(8, true); break;
+    default: K3_FAIL(K3HIP_EUNSUPPORTED, "mla absorb: qk_nope=%d padded to %d", QN, QNP);
     }
 #undef K3_ABS
     K3_LAUNCHED();
@@ -250,9 +273,8 @@ __global__ void mla_norm_kernel(long ldc, float eps, NormJob j0, NormJob j1, lon
     }
 }
 
-// qcat[b][h] = [ sum over planes p of A2[pB+b][h] (the absorbed W_UK_h^T q_nope, kv_lora floats) |
-// q_rope(b,h) ], from the absorb product's planes and the fp32 q.
-__global__ void mla_qcat_kernel(const float *__restrict__ A2, int planes, const float *__restrict__ q, int B,
+// qcat[b][h] = [ A2[b][h] (the absorbed W_UK_h^T q_nope, kv_lora floats) | q_rope(b,h) ].
+__global__ void mla_qcat_kernel(const float *__restrict__ A2, const float *__restrict__ q, int B,
                                 int H, int QN, int QR, int KL, float *__restrict__ qcat)
 {
     const int W = KL + QR, QH = QN + QR;
@@ -261,10 +283,7 @@ __global__ void mla_qcat_kernel(const float *__restrict__ A2, int planes, const 
          i += (size_t)gridDim.x * blockDim.x) {
         const size_t bh = i / W;
         const int c = (int)(i % W);
-        float v = c < KL ? A2[i] : q[bh * QH + QN + (c - KL)];
-        if (c < KL)
-            for (int p = 1; p < planes; p++) v += A2[(size_t)p * n + i];
-        qcat[i] = v;
+        qcat[i] = c < KL ? A2[i] : q[bh * QH + QN + (c - KL)];
     }
 }
 
@@ -427,10 +446,9 @@ extern "C" int k3hip_mla_upload(const K3MlaW *w, const K3Cfg *c, k3hip_mla_weigh
             K3_FAIL(K3HIP_ENOMEM, "k3hip_mla_upload: device copy of %zu bytes", u.bytes);
         }
     }
-    // W_UK^T per head for the absorb kernel (qk_nope <= 256; wider heads keep the batched
-    // library GEMM on kv_b itself)
-    d->QNP = (d->QN + 31) / 32 * 32;
-    if (d->QNP <= 256) {
+    // W_UK^T per head for the absorb kernel
+    d->QNP = absorb_row(d->QN);
+    {
         const size_t n = H * d->KL * d->QNP;
         if (device_alloc(&d->ukt, n * 2) != hipSuccess) {
             (void)hipGetLastError();
@@ -488,9 +506,7 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     // attention in one pass over the cache (kda_mla_attn.hip) where the shape fits it, else
     // as two strided-batched fp32 GEMMs around the softmax
     const bool fused = mla_attention_supported(H, KL, CW) && !((uintptr_t)cache & 15) && !(QN & 3) && VH <= 128;
-    // planes of the absorb product: one from the absorb kernel, three from the library GEMM
-    const int planes = w->ukt ? 1 : 3;
-    // scratch: q_a kv_a g projections [B][ld1] | q_a normed | q | q split | absorb planes | qcat |
+    // scratch: q_a kv_a g projections [B][ld1] | q_a normed | q | absorb product | qcat |
     //          scores or the fused attention's workspace | chat | chat split | W_UV planes (qcat,
     //          the chat split and the W_UV planes only without the fused attention) | o | split-K partials
     const int N1 = QL + CW + (w->gate ? HV : 0);
@@ -501,8 +517,7 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     const size_t wsf = std::max({gemm_rows_ws_floats(B, N1, E), np1 > 1 ? (size_t)np1 * std::min(64, B) * N1 : 0,
                                  gemm_rows_ws_floats(B, H * QH, QL), gemm_rows_ws_floats(B, E, HV)});
     size_t sizes[] = {(size_t)B * ld1 * 4, (size_t)B * QL * 4, (size_t)B * H * QH * 4,
-                      w->ukt ? 0 : (size_t)3 * B * H * QH * 2, (size_t)planes * B * H * CW * 4,
-                      fused ? 0 : (size_t)B * H * CW * 4,
+                      (size_t)B * H * CW * 4, fused ? 0 : (size_t)B * H * CW * 4,
                       fused ? mla_attention_ws_bytes(B, H, KL, Tn) : (size_t)B * H * Tn * 4,
                       (size_t)B * H * KL * 4, fused ? 0 : (size_t)3 * B * H * KL * 2,
                       fused ? 0 : (size_t)3 * B * HV * 4, (size_t)B * HV * 4, wsf * 4};
@@ -517,20 +532,19 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     if (rc) return rc;
     char *base = (char *)buf.p;
     float *C1 = (float *)(base + off[0]), *qn = (float *)(base + off[1]), *q = (float *)(base + off[2]);
-    uint16_t *qs3 = (uint16_t *)(base + off[3]);
-    float *A2 = (float *)(base + off[4]), *qcat = (float *)(base + off[5]), *S = (float *)(base + off[6]);
-    float *chat = (float *)(base + off[7]);
-    uint16_t *ch3 = (uint16_t *)(base + off[8]);
-    float *O2 = (float *)(base + off[9]), *o = (float *)(base + off[10]), *ws = (float *)(base + off[11]);
+    float *A2 = (float *)(base + off[3]), *qcat = (float *)(base + off[4]), *S = (float *)(base + off[5]);
+    float *chat = (float *)(base + off[6]);
+    uint16_t *ch3 = (uint16_t *)(base + off[7]);
+    float *O2 = (float *)(base + off[8]), *o = (float *)(base + off[9]), *ws = (float *)(base + off[10]);
     const uint16_t *kvb = (const uint16_t *)w->kv_b;
 
     // q_a, kv_a and g in one pass over their weights (fp32 x split in registers);
     // q = q_b(rmsnorm(q_a x)); latent + rope = kv_a x, the latent rmsnorm'd into the cache
     if ((rc = gemm_rows_even(B, N1, E, x, E, (const uint16_t *)w->xin, C1, ld1, st, ws, wsf))) return rc;
-    // the two rmsnorms: with the absorb kernel and an unsplit q_b product, the q_b GEMV
+    // the two rmsnorms: with the fused attention and an unsplit q_b product, the q_b GEMV
     // normalises q_a as it reads it and the absorb launch writes the new latent row;
     // otherwise one launch writes qn and the cache row
-    const bool fold_norms = fused && w->ukt && gemm_rows_splits(H * QH, QL) == 1 && !((uintptr_t)w->q_a_norm & 15);
+    const bool fold_norms = fused && gemm_rows_splits(H * QH, QL) == 1 && !((uintptr_t)w->q_a_norm & 15);
     if (!fold_norms) {
         hipLaunchKernelGGL(mla_norm_kernel, dim3(B, 2), dim3(256), 0, st, ld1, w->eps,
                            NormJob{C1, QL, QL, w->q_a_norm, qn, nullptr},
@@ -542,21 +556,10 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     else
         rc = gemm_rows(B, H * QH, QL, qn, QL, (const uint16_t *)w->q_b, q, (long)H * QH, st, ws, wsf);
     if (rc) return rc;
-    // absorb: per head h, q (B x QN) . W_UK_h (QN x KL); the library GEMM takes q as split rows
-    if (w->ukt) {
-        if ((rc = mla_absorb(B, H, QH, QN, w->QNP, KL, CW, q, (long)H * QH, (const uint16_t *)w->ukt, A2,
-                             (long)H * CW,
-                             LatRow{fold_norms ? C1 + QL : nullptr, ld1, w->kv_a_norm, w->eps, cache, (long)cap, pos, B},
-                             st)))
-            return rc;
-    } else {
-        if ((rc = split_rows3(q, qs3, B, H * QH, st))) return rc;
-        GemmDesc ga;
-        ga.M = 3 * B; ga.N = KL; ga.K = QN; ga.ab_dtype = K3HIP_BF16; ga.c_dtype = K3HIP_F32; ga.b_trans = false;
-        ga.lda = (long)H * QH; ga.ldb = KL; ga.ldc = (long)H * CW; ga.batch = H;
-        ga.sa = QH; ga.sb = (long)(QN + VH) * KL; ga.sc = CW;
-        if ((rc = gemm(ga, qs3, kvb, A2, st))) return rc;
-    }
+    // absorb: per head h, q (B x QN) . W_UK_h (QN x KL)
+    if ((rc = mla_absorb(B, H, QH, QN, w->QNP, KL, CW, q, (long)H * QH, (const uint16_t *)w->ukt, A2, (long)H * CW,
+                         LatRow{fold_norms ? C1 + QL : nullptr, ld1, w->kv_a_norm, w->eps, cache, (long)cap, pos, B}, st)))
+        return rc;
     // o_proj as two K-ranges adds into `out`, zeroed by the kernel before it (no reduction
     // launch); atomics on ordinary device memory only
     const bool oz = gemm_rows_splits(E, HV) == 2 && coarse_device_mem(out);
@@ -564,15 +567,15 @@ extern "C" int k3hip_mla_decode(const k3hip_mla_weights *w, int B, int pos, int 
     if (fused) {
         // the query rows formed inside the attention from A2 and q; the ranges merged, W_UV and
         // the output gate applied in the launch after it (kda_mla_attn.hip)
-        if ((rc = mla_attention(B, H, KL, CW, Tn, cap, 1.0f / sqrtf((float)QH), A2, planes, q, QN, cache, kvb, VH, gl, ld1,
+        if ((rc = mla_attention(B, H, KL, CW, Tn, cap, 1.0f / sqrtf((float)QH), A2, q, QN, cache, kvb, VH, gl, ld1,
                                 o, oz ? out : nullptr, oz ? (size_t)B * E : (size_t)0, chat, S,
                                 mla_attention_ws_bytes(B, H, KL, Tn), st)))
             return rc;
         return gemm_rows(B, E, HV, o, HV, (const uint16_t *)w->o, out, E, st, ws, wsf, oz);
     }
     {
-        hipLaunchKernelGGL(mla_qcat_kernel, dim3(mla_grid((size_t)B * H * CW)), dim3(256), 0, st, A2, planes, q,
-                           B, H, QN, QR, KL, qcat);
+        hipLaunchKernelGGL(mla_qcat_kernel, dim3(mla_grid((size_t)B * H * CW)), dim3(256), 0, st, A2, q, B, H,
+                           QN, QR, KL, qcat);
         K3_LAUNCHED();
         // scores S_b [H][Tn] = qcat_b [H][CW] . cache_b[0..Tn)^T, per sequence
         GemmDesc gs;

@@ -85,12 +85,11 @@ struct AtGeom {
     int H, CW, KL;
 };
 
-// Where the query rows come from: qcat[b][h] = [sum over planes p of A2[pB+b][h] (one plane from
-// the absorb kernel, three from the batched library GEMM on q's split rows; KL floats) |
+// Where the query rows come from: qcat[b][h] = [A2[b][h] (the absorb product, KL floats) |
 // q_rope(b, h) (q [B][H][QH] at column QN)], formed while the q fragments are loaded.
 struct AtQ {
     const float *A2, *q;
-    int planes, B, QN, QH;
+    int QN, QH;
 };
 
 __device__ __forceinline__ void split2(float a, float b, bf16x2 &hi, bf16x2 &lo)
@@ -184,11 +183,7 @@ __global__ __launch_bounds__(AT_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
                     const int cc = c + e;
                     f4 v = f4{0.0f, 0.0f, 0.0f, 0.0f};
                     if (ok && cc < CW) {
-                        if (cc < KL) {
-                            v = *reinterpret_cast<const f4 *>(a2 + cc);
-                            for (int p = 1; p < qs.planes; p++)
-                                v += *reinterpret_cast<const f4 *>(a2 + (size_t)p * qs.B * H * CW + cc);
-                        } else v = *reinterpret_cast<const f4 *>(qr + cc);
+                        v = *reinterpret_cast<const f4 *>((cc < KL ? a2 : qr) + cc);
                     }
                     x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
                 }
@@ -616,7 +611,7 @@ bool mla_attention_supported(int H, int KL, int CW)
     return at_geom(H, KL, CW, g);
 }
 
-int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, int planes, const float *q,
+int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, const float *A2, const float *q,
                   int QN, const float *cache, const uint16_t *kvb, int VH, const float *gate, long ldg, float *o, float *zout, size_t zn,
                   float *chat, void *ws, size_t ws_bytes, hipStream_t st)
 {
@@ -631,7 +626,7 @@ int mla_attention(int B, int H, int KL, int CW, int Tn, int cap, float scale, co
         ((uintptr_t)q & 15) || (QN & 3) || (KL & 7) || ((uintptr_t)kvb & 15) || ((uintptr_t)chat & 15) ||
         VH < 1 || VH > 16 * (AO_NT / 64))
         K3_FAIL(K3HIP_EINVAL, "mla attention: workspace %zu < %zu bytes, or a misaligned buffer", ws_bytes, need);
-    const AtQ qs{A2, q, planes, B, QN, QH};
+    const AtQ qs{A2, q, QN, QH};
     const size_t r = (size_t)B * nsplit * H;
     float *pctx = (float *)ws;
     float *pm = (float *)((char *)ws + ((r * KL * 4 + 255) & ~(size_t)255));
