@@ -17,8 +17,11 @@
 // give every CU one, 128 x 128 for bf16 rows where those do), four waves in 2 x 2, K in steps of
 // 64. Weights and bf16 rows come by direct-to-LDS buffer loads into 2, 3 or 5 buffers, each requested
 // 1, 2 or 4 steps before it is read; fp32 rows go through registers one step ahead and are
-// split as they are put in LDS (two buffers). 64-80 KiB of LDS; where two workgroups share a
-// CU, one's barrier and load waits hide behind the other's products. Rows are 128 bytes, the
+// split as they are put in LDS (two buffers). Loads come back in order, so the wait for a step's
+// fp32 rows is one for all but the newest step's weights, and a third buffer is the last that
+// helps (64 x 64 tiles: five 91.6 us, three 90.4 for the 100-token layer at hidden 2048, 16 x 128).
+// 56-80 KiB of LDS; where two workgroups share a CU, one's barrier and load waits hide behind the
+// other's products. Rows are 128 bytes, the
 // 16-byte chunk index XORed with (row & 7) ^ ((row >> 3) & 1): 16-lane fragment reads fall on
 // distinct banks. The weight is the MFMA's first operand, so a lane ends with four adjacent
 // columns of one row: 16-byte stores. A column tile's row tiles run on one XCD (workgroup id
@@ -270,7 +273,7 @@ int launch(MidArgs &a, int M, int K, const void *A, long lda, hipStream_t st)
     }
     // 64 rows, and 128 columns once those tiles give every CU one; 64 below
     if (wide * ((M + 63) / 64) >= ncu) return launch_tile<AM, 64, 128, 3>(a, M, K, A, lda, st);
-    return launch_tile<AM, 64, 64, 5>(a, M, K, A, lda, st);
+    return launch_tile<AM, 64, 64, AM == MID_A_16 ? 5 : 3>(a, M, K, A, lda, st);
 }
 
 }  // namespace
