@@ -318,12 +318,16 @@ static bool chunk_gate_ok(float lb) { return lb < 0.0f && fabsf(lb) * 15.0f <= 8
 
 // Where k3hip_kda_layer_dev runs its bf16 projections. Fewer than 33 tokens: the double products
 // of kda_proj.hip, no slower there and more accurate (hidden 1024, 8 x 64 heads T = 24: 40 us
-// against 50; hidden 4096, 32 x 128: 163 | 153, but T = 36 already 213 | 155). Then
-// kda_mid.hip up to MID_DEV_MACS products of the input projections (hidden 4096, 32 x 128 heads
-// T = 333: 775 -> 249 us, T = 3000 (2.0e11) 1622 -> 1497 us; T = 8192 (5.6e11) 3933 | 4104), then
-// the 256 x 256 tiles of kda_mm.hip on 2T split rows.
+// against 50; hidden 4096, 32 x 128: 163 | 153, but T = 36 already 213 | 155). Then kda_mid.hip up
+// to this many products of the input projections, then the 256 x 256 tiles of kda_mm.hip on 2T split
+// rows (the same bits). Those do a product faster, but pay for idle tiles and for writing, reading
+// and adding the halves, which weighs the more the narrower the layer. Layer times, mid | mm: hidden
+// 4096, 32 x 128 heads T = 333 (2.3e10) 256 us | 732, T = 1500 (1.0e11) 784 | 883, T = 2200 (1.5e11)
+// 1198 | 1402, T = 3000 (2.0e11) 1551 | 1506, T = 5800 (3.9e11) 3033 | 2523; hidden 7168 T = 1600 (1.9e11)
+// 1412 | 1456; hidden 3072 T = 5000 (2.5e11) 2120 | 2028; hidden 2048, 48 x 128 T = 6000 (3.0e11) 2841 |
+// 2895; hidden 1024, 32 x 128 T = 12000 (2.0e11) 2286 | 2665.
 constexpr int MID_DEV_T = 33;
-constexpr double MID_DEV_MACS = 4e11;
+static double mid_dev_macs(int hidden) { return hidden > 2048 ? 2e11 : 4e11; }
 
 extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out, const float *x,
                                    float *state, void *stream)
@@ -376,7 +380,7 @@ extern "C" int k3hip_kda_layer_dev(const k3hip_kda_weights *w, int T, float *out
     // double-accumulating products of kda_proj.hip.
     const bool mfma = w->wdt == K3_WBF16 && T >= MID_DEV_T && E % 64 == 0 && D % 64 == 0 && P % 64 == 0 &&
                       ((uintptr_t)x & 15) == 0;
-    const bool big = mfma && (double)T * (4.0 * P + D + H) * E > MID_DEV_MACS;
+    const bool big = mfma && (double)T * (4.0 * P + D + H) * E > mid_dev_macs(E);
     StreamBuf sbuf;
     uint16_t *xs = nullptr;
     float *C2 = nullptr;
@@ -772,7 +776,7 @@ static int layer_decode_impl(const k3hip_kda_weights *w, int B, float *out, cons
                    *Wfb = (const uint16_t *)w->f_b_f, *Wo = (const uint16_t *)w->o_f;
 
     // 1 projections: the fp32 rows against bf16 weights, each weight read once for all B
-    //   (kda_rows.hip: x split into bf16 hi + lo in registers); q, k, v, f_a and the beta
+    //   (kda_rows.hip: x split into three bf16 parts in registers); q, k, v, f_a and the beta
     //   logits in one pass over their concatenated weights; the output gate left as split-K
     //   planes that the step kernel adds
     if ((rc = gemm_rows_with_part(B, E, x, E, NI, Win, Cin, ldi, (int)P, Wg, glp, st, ws, wsf))) return rc;

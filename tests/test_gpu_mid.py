@@ -100,14 +100,14 @@ def test_short_prefill_projections_vs_oracle(gpu, hidden, H, D, Ts, dev):
 
 
 def test_split_rows_and_tiles_give_the_same_bits(gpu):
-    """The full-accuracy layer's longest prefills (from 4e11 products of the input projections) run
-    kda_mm.hip on 2T split rows and add the halves, shorter ones kda_mid.hip with an accumulator
-    per half: a sequence in one call of the first kind and in two of the second (chunk boundaries do
-    not move) is the same bits."""
+    """The full-accuracy layer's longest prefills (at this width from 2e11 products of the input
+    projections) run kda_mm.hip on 2T split rows and add the halves, shorter ones kda_mid.hip with
+    an accumulator per half: a sequence in one call of the first kind and in two of the second
+    (chunk boundaries do not move) is the same bits."""
     import torch
-    hidden, H, D, K, T = 4096, 32, 128, 4, 6016
+    hidden, H, D, K, T = 4096, 32, 128, 4, 3072
     P = H * D
-    assert T / 2 * (4 * P + D + H) * hidden < 4e11 < T * (4 * P + D + H) * hidden and T // 2 % 64 == 0
+    assert T / 2 * (4 * P + D + H) * hidden < 2e11 < T * (4 * P + D + H) * hidden and T // 2 % 64 == 0
     cfg = ko.make_cfg(hidden, H, D, K, -5.0, 1e-5)
     dw = gpu.DeviceWeights(layer_weights(np.random.default_rng(9), hidden, H, D, K).w, cfg, gpu.UPLOAD_DEV)
     x = torch.randn((T, hidden), device="cuda", generator=torch.Generator(device="cuda").manual_seed(9))
