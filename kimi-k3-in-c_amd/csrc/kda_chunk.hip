@@ -137,8 +137,9 @@ __device__ __forceinline__ void store_cpl(float *p, const float (&v)[CPL])
 // the inputs (phase 1 at T=8192, H=32, D=128 -5 us with the compiler's nontemporal stores, and
 // the core step 0.5355 -> 0.5333 ms with this policy; ordinary stores 0.533 against 0.521). A
 // smaller one (KEEP) is stored ordinarily and found in that cache: T=701, 6 x 64 heads 35.1 ->
-// 32.0 us; T=2048, 32 x 128 (151 MB) 144.3 -> 140.6; T=5000, 8 x 128 188 -> 167; the two meet
-// at 250 MB (T=3400, 32 x 128: 233.3 | 233.8). They are compiler-visible stores, so the wait states
+// 32.0 us; T=2048, 32 x 128 (151 MB) 144.3 -> 140.6; T=5000, 8 x 128 188 -> 167; one
+// chunk of 96 x 128 38.8 -> 36.9, but of 28 to 32 x 128 up to 0.8 the other way (27.7 | 28.5); the
+// two meet at 250 MB (T=3400, 32 x 128: 233.3 | 233.8). They are compiler-visible stores, so the wait states
 // a store needs (an MFMA result as data, a VALU overwrite of its data registers) are inserted
 // as for any other.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t ws_rsrc(char *blk, size_t bytes)
